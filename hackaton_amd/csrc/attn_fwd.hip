@@ -611,28 +611,51 @@ __global__ __launch_bounds__(fwd::NT, 1) void fwd_kernel(
 
 // --------------------------------------------------------------------------------------------
 // Forward for many work items: 4 waves per work item (one per query strip, each over all of the
-// item's key tiles), 64 KB of LDS, so two work-groups share a CU. The two waves of a SIMD then
-// come from different work items with their own barriers: one's MFMAs overlap the other's
-// softmax without any phase arrangement, one item's start (loads) and end (stores) overlap the
-// other's tiles, and no item merges halves at its end. Used when the plan has enough items to
-// give every CU two (kFwdLeanMinItems).
+// item's key tiles), three work-groups per CU. The three waves of a SIMD come from different work
+// items with their own barriers: one's MFMAs overlap the others' softmax and waits without any
+// phase arrangement, one item's start (loads) and end (stores) overlap the others' tiles, and no
+// item merges halves at its end.
+//
+// Three waves per SIMD leave 168 registers and 53 KB of LDS each: 32-key tiles (16 scores per
+// lane) in a ring of three stages, the copies two tiles ahead, one barrier per tile. A tile's rows
+// are stored in groups of 4 (1 KB, one copy instruction) 1088 bytes apart, chunk c of row r at
+// c ^ (r & 3): the 64-byte shift from group to group and the two XOR bits spread 16 rows of K
+// over the 16 chunk columns, and the transposed V reads (4 rows x 32 bytes of columns j and
+// j + 64) over all 64 banks, while all but two address bits stay immediates: 6 address registers
+// instead of 16.
+//
+// What bounds it: at documents of thousands of tokens the matrix cores' sustained rate on real
+// data (two documents of 8192 tokens, 28/4 heads, bf16: 883 us = 1090 TFLOP/s, where an 8192^3
+// library product reaches 1390 on the same card; the MFMAs alone take 588 us, everything else
+// 493 us); at documents of a few hundred tokens the first loads and the last stores of each item
+// and HBM. Against two work-groups of 64-key tiles in two stages, 256 registers (interleaved
+// runs, one card): 8192-token documents 897 -> 883 us; 32768 tokens of 32 to 1740, 28/4 heads,
+// bf16 286 -> 263 us; 16384 tokens of 8 to 511, 12/2 heads, bf16 45.2 -> 41.7 us; 8192 tokens of
+// 16 to 512, 12/2 heads, fp16 24.5 -> 23.9 us. The same tiles in a ring of four stages, which
+// leaves two work-groups a CU, take 938 / 286 / 48 / 25 us.
 // --------------------------------------------------------------------------------------------
 namespace fwdl {
 constexpr int NW = fwd::NS;     // waves = query strips
 constexpr int NT = NW * 64;
-constexpr int BN = fwd::BN, D = fwd::D, TILE = fwd::TILE;
-constexpr int STAGE = 2 * TILE;  // K, V of one 64-key tile
-constexpr int BM = fwd::BM;
-static_assert(BM * D <= STAGE, "the Q tile fits in one stage");
+constexpr int BN = 32;          // keys per tile
+constexpr int D = fwd::D, BM = fwd::BM;
+constexpr int GRP = 4 * D + 32;       // halfs from one group of 4 rows to the next
+constexpr int TILE = BN / 4 * GRP;    // halfs of a K or V tile
+constexpr int STAGE = 2 * TILE;       // K, V of one tile
+constexpr int NSTAGE = 3;
+constexpr int PER_CU = 3;             // work-groups per CU
+static_assert(BM / 4 * GRP <= (NSTAGE - 1) * STAGE, "the Q tile fits in stages 1 and 2");
+static_assert(PER_CU * NSTAGE * STAGE * 2 <= 160 * 1024, "LDS of three work-groups");
+static_assert(BN / 4 * 2 == 4 * NW, "copy map: 4 row groups per wave and tile pair K, V");
 }  // namespace fwdl
 
 template <class E>
-__global__ __launch_bounds__(fwdl::NT, 2) void fwd_lean_kernel(
+__global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
     const int4* __restrict__ items, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int hq, int hkv,
     uint16_t* __restrict__ o, float* __restrict__ lse, int n_tokens, float scale_log2) {
   using namespace fwdl;
-  __shared__ __attribute__((aligned(16))) uint16_t smem_raw[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) uint16_t smem_raw[NSTAGE * STAGE];
   lds_u16* smem = (lds_u16*)smem_raw;
 
   const int4 it = items[blockIdx.x];
@@ -654,46 +677,47 @@ __global__ __launch_bounds__(fwdl::NT, 2) void fwd_lean_kernel(
   const bool q_valid = my_q < q_end;
   const int ws = __builtin_amdgcn_readfirstlane(strip);
   const int wq0_u = __builtin_amdgcn_readfirstlane(wq0);
+  const int n_tiles = (q_end - doc_start + BN - 1) / BN;
 
-  const int kv_end = q_end;
-  const int n_tiles = (kv_end - doc_start + BN - 1) / BN;
-
-  // Copy of tile t (K and V) into a stage: wave s moves row groups 4 s .. 4 s + 3 (4 rows each)
-  // of both tensors, 8 instructions; lane i lands in chunk slot i & 15 of row i >> 4 of the group
-  // and fetches logical chunk (i & 15) ^ swz16(row). Rows past the document end read as zeros.
-  int coff[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = 4 * (4 * strip + j) + (lane >> 4);
-    coff[j] = (r * (int)kvrow + 8 * ((lane & 15) ^ swz16(r))) * 2;
-  }
-  auto copy_tile = [&](int t, int stage) {
-    const int row0 = doc_start + t * BN;
-    const long base = (long)row0 * kvrow + kvh * D;
-    const long bytes = ((long)(doc_end - row0 - 1) * kvrow + D) * 2;
-    const uint32_t dst = lds_addr(smem + stage * STAGE);
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      const u32x4 r = make_rsrc4((x ? v : k) + base, bytes);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        dma16_opaque(r, dst + (x * TILE + 4 * (4 * ws + j) * D) * 2, coff[j]);
-    }
+  // Copies of the tiles, in tile order: wave s moves row groups 2 s and 2 s + 1 of K and of V, 4
+  // instructions; lane i lands in chunk slot i & 15 of row i >> 4 of the group and fetches the
+  // chunk that belongs there. Rows past the document end read as zeros (masked keys, zero P).
+  const int c_row = lane >> 4;
+  const int coff = ((8 * ws + c_row) * (int)kvrow + 8 * ((lane & 15) ^ c_row)) * 2;
+  const int coff4 = 4 * (int)kvrow * 2;
+  const uint16_t* kp = k + (long)doc_start * kvrow + kvh * D;
+  const uint16_t* vp = v + (long)doc_start * kvrow + kvh * D;
+  long left = ((long)(doc_end - doc_start - 1) * kvrow + D) * 2;  // bytes from kp to the end
+  const long step = (long)BN * kvrow;
+  auto copy_next = [&](uint32_t dst) {
+    const u32x4 rk = make_rsrc4(kp, left), rv = make_rsrc4(vp, left);
+    dst += 2 * ws * GRP * 2;
+    dma16_opaque(rk, dst, coff);
+    dma16_opaque(rk, dst + GRP * 2, coff + coff4);
+    dma16_opaque(rv, dst + TILE * 2, coff);
+    dma16_opaque(rv, dst + (TILE + GRP) * 2, coff + coff4);
+    kp += step;
+    vp += step;
+    left -= step * 2;
   };
 
-  int koff[8], toff[4][2];
+  // Read offsets (halfs) inside a tile. K (A operand of S^T): row perm32(l32), chunk 2 kk + hi.
+  // V^T: row 8 hi + 2 (src >> 2) + e (+ 16 c), chunk 8 (grp & 1) + 2 db + (sg >> 1): registers
+  // [8 c, 8 c + 8) of accumulator db then hold d = 16 db + 64 c + 8 hi + 0..7.
+  int koff[2], toff[2][2];
   {
-    const int r = perm32(l32), f = swz16(r);
+    const int r = perm32(l32);
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) koff[kk] = r * D + 8 * ((2 * kk + hi) ^ f);
+    for (int p = 0; p < 2; ++p)
+      koff[p] = (r >> 2) * GRP + (r & 3) * D + 8 * ((2 * p + hi) ^ (r & 3));
     const int sg = (((src & 3) & 1) << 1) | ((src & 3) >> 1);
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const int rr = 8 * hi + 2 * (src >> 2) + e;
-        const int lc = 2 * (grp & 1) + 4 * db + (sg >> 1);
-        toff[db][e] = rr * D + 8 * (lc ^ swz16(rr)) + 4 * (sg & 1);
+        toff[p][e] = (rr >> 2) * GRP + (rr & 3) * D +
+                     8 * (8 * (grp & 1) + ((2 * p + (sg >> 1)) ^ (rr & 3))) + 4 * (sg & 1);
       }
   }
 
@@ -703,34 +727,25 @@ __global__ __launch_bounds__(fwdl::NT, 2) void fwd_lean_kernel(
   for (int db = 0; db < 4; ++db) oacc[db] = f32x16{};
   float m_run = -INFINITY, l_run = 0.f;
 
-  // S^T of one 64-key tile (K at `kb`): 16 MFMAs, each K operand read 4 MFMAs ahead.
-  auto s_tile = [&](const lds_u16* kb, f32x16(&s)[2]) {
-    s[0] = f32x16{};
-    s[1] = f32x16{};
+  // S^T of one tile (K at `kb`): 8 MFMAs, each K operand read 4 MFMAs ahead.
+  auto s_tile = [&](const lds_u16* kb, f32x16& s) {
+    s = f32x16{};
+    auto k_read = [&](int i) { return ld128(kb + koff[i & 1] + 32 * (i >> 1)); };
     u32x4 ka[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ka[i] = ld128(kb + koff[i >> 1] + 32 * (i & 1) * D);
+    for (int i = 0; i < 4; ++i) ka[i] = k_read(i);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int kk = i >> 1, b = i & 1;
-      s[b] = E::mfma(ka[i & 3], qf[kk], s[b]);
-      if (i + 4 < 16) ka[i & 3] = ld128(kb + koff[(i + 4) >> 1] + 32 * ((i + 4) & 1) * D);
+    for (int i = 0; i < 8; ++i) {
+      s = E::mfma(ka[i & 3], qf[i], s);
+      if (i + 4 < 8) ka[i & 3] = k_read(i + 4);
     }
-    VA_SCHED(kSchedDsRead, 4);
-#pragma unroll
-    for (int i = 0; i < 12; ++i) {
-      VA_SCHED(kSchedMfma, 1);
-      VA_SCHED(kSchedDsRead, 1);
-    }
-    VA_SCHED(kSchedMfma, 4);
   };
-  // Mask, online softmax and O^T += V^T P^T of tile t (V at `vb`), as in the two-half kernel.
-  auto pv_tile = [&](const lds_u16* vb, int t, f32x16(&s)[2]) {
-    const int kv0 = doc_start + t * BN;
-    auto v_read = [&](int i) {
-      const int b = i >> 3, c = (i >> 2) & 1, db = i & 3;
-      const lds_u16* p = vb + (32 * b + 16 * c) * D;
-      const u32x2 x = ldtr(p + toff[db][0]), y = ldtr(p + toff[db][1]);
+  // Mask, online softmax and O^T += V^T P^T of the tile of keys from kv0 (V at `vb`).
+  auto pv_tile = [&](const lds_u16* vb, int kv0, f32x16& s) {
+    auto v_read = [&](int i) {  // i = (c, db) in MFMA order
+      const int c = i >> 2, db = i & 3;
+      const lds_u16* p = vb + 4 * c * GRP + 32 * (db >> 1);
+      const u32x2 x = ldtr(p + toff[db & 1][0]), y = ldtr(p + toff[db & 1][1]);
       return u32x4{x[0], x[1], y[0], y[1]};
     };
     u32x4 va[4];
@@ -739,16 +754,12 @@ __global__ __launch_bounds__(fwdl::NT, 2) void fwd_lean_kernel(
     if (kv0 + BN - 1 > wq0_u) {
       const int lim = my_q - kv0;
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-          if (32 * b + reg_row(j, hi) > lim) s[b][j] = -INFINITY;
+      for (int j = 0; j < 16; ++j)
+        if (reg_row(j, hi) > lim) s[j] = -INFINITY;
     }
     float mt = -INFINITY;
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) mt = fmaxf(mt, s[b][j]);
+    for (int j = 0; j < 16; ++j) mt = fmaxf(mt, s[j]);
     mt = max_with_other_half(mt) * scale_log2;
     if (__builtin_amdgcn_ballot_w64(mt > m_run + fwd::kRescaleLog2)) {
       const float m_new = fmaxf(m_run, mt);
@@ -759,84 +770,90 @@ __global__ __launch_bounds__(fwdl::NT, 2) void fwd_lean_kernel(
       for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
     }
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
-    float rs = 0.f;
-    u32x4 pf[2][2];
+    float rs[2] = {0.f, 0.f};
+    u32x4 pf[2];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int c = 0; c < 2; ++c) {
+      float p[8];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        float p[8];
+      for (int e = 0; e < 8; ++e) p[e] = fast_exp2(fmaf(s[8 * c + e], scale_log2, -m_use));
+      pf[c] = pack8_tr<E>(p);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) p[e] = fast_exp2(fmaf(s[b][8 * c + e], scale_log2, -m_use));
-        pf[b][c] = pack8_tr<E>(p);
+      for (int w = 0; w < 4; ++w) rs[c] = E::sum2(pf[c][w], rs[c]);
+    }
+    l_run += rs[0] + rs[1];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) rs = E::sum2(pf[b][c][w], rs);
-      }
-    l_run += rs;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int b = i >> 3, c = (i >> 2) & 1, db = i & 3;
-      oacc[db] = E::mfma(va[i & 3], pf[b][c], oacc[db]);
-      if (i + 4 < 16) va[i & 3] = v_read(i + 4);
+    for (int i = 0; i < 8; ++i) {
+      oacc[i & 3] = E::mfma(va[i & 3], pf[i >> 2], oacc[i & 3]);
+      if (i + 4 < 8) va[i & 3] = v_read(i + 4);
     }
   };
 
-  // Q (32 KB) into the second stage, tile 0 into the first; every lane reads its query's row.
+  // Q (32 row groups) into stages 1 and 2, tile 0 into stage 0; every lane reads its query's row.
   {
-    const long bytes = ((long)(doc_end - q0 - 1) * qrow + (long)(h + 1) * D) * 2;
-    const u32x4 rq = make_rsrc4(q + (long)q0 * qrow, bytes);
+    const long bytes = ((long)(doc_end - q0 - 1) * qrow + D) * 2;
+    const u32x4 rq = make_rsrc4(q + (long)q0 * qrow + h * D, bytes);
+    const int off = ((32 * ws + c_row) * (int)qrow + 8 * ((lane & 15) ^ c_row)) * 2;
+    const uint32_t dst = lds_addr(smem + STAGE + 8 * ws * GRP);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int r = 32 * strip + 4 * j + (lane >> 4);
-      dma16_opaque(rq, lds_addr(smem + STAGE + (32 * ws + 4 * j) * D),
-                   (r * (int)qrow + h * D + 8 * ((lane & 15) ^ swz16(r))) * 2);
-    }
+    for (int j = 0; j < 8; ++j) dma16_opaque(rq, dst + j * GRP * 2, off + 4 * j * (int)qrow * 2);
   }
-  copy_tile(0, 0);
+  copy_next(lds_addr(smem));
   wait_vmcnt<0>();
   __syncthreads();
   {
-    const int r = 32 * strip + l32, f = swz16(r);
+    const lds_u16* qt = smem + STAGE + (8 * strip + (l32 >> 2)) * GRP + (l32 & 3) * D;
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) qf[kk] = ld128(smem + STAGE + r * D + 8 * ((2 * kk + hi) ^ f));
+    for (int kk = 0; kk < 8; ++kk)
+      qf[kk] = ld128(qt + 8 * ((2 * (kk & 1) + hi) ^ (l32 & 3)) + 32 * (kk >> 1));
   }
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) settle(qf[kk]);
-  __syncthreads();  // every wave holds its Q before the loop overwrites the second stage
-  // A strip past the document's end (the last item of a document whose length is not a multiple
-  // of 128) has no query to compute: its wave only copies and meets the barriers, and leaves its
-  // SIMD to the other work-group's wave.
-  const bool strip_live = wq0_u < q_end;
-  auto visible = [&](int t) { return strip_live && doc_start + t * BN <= wq0_u + 31; };
-  for (int t = 0; t < n_tiles; ++t) {
-    const int stage = t & 1;
-    // The next tile's copies go out after this tile's S^T MFMAs (the wave waits for S anyway).
-    if (visible(t)) {
-      f32x16 s[2];
-      s_tile(smem + stage * STAGE, s);
-      if (t + 1 < n_tiles) copy_tile(t + 1, stage ^ 1);
-      pv_tile(smem + stage * STAGE + TILE, t, s);
-    } else if (t + 1 < n_tiles) {
-      copy_tile(t + 1, stage ^ 1);
-    }
-    wait_vmcnt<0>();  // this wave's copies of the next tile have landed in LDS
+  __syncthreads();  // every wave holds its Q before the ring overwrites it
+  // A strip computes the tiles up to its diagonal; past them, and in a strip past the document's
+  // end (the last item of a document whose length is not a multiple of 128), its wave only copies
+  // and meets the barriers, and leaves its SIMD to the other work-groups' waves.
+  const int n_live = wq0_u < q_end ? min((wq0_u + 31 - doc_start) / BN + 1, n_tiles) : 0;
+  if (1 < n_tiles) copy_next(lds_addr(smem + STAGE));
+  int stage = 0;
+  auto next = [&](int t) {
+    // This wave's copies of tile t + 1 have landed in LDS; those of tile t + 2 stay in flight.
+    if (t + 2 < n_tiles) wait_vmcnt<4>();
+    else wait_vmcnt<0>();
     __syncthreads();
+    stage = stage == NSTAGE - 1 ? 0 : stage + 1;
+  };
+  auto copy_ahead = [&](int t) {  // tile t + 2, into the stage that tile t - 1 was last read from
+    if (t + 2 < n_tiles) copy_next(lds_addr(smem + (stage == 0 ? NSTAGE - 1 : stage - 1) * STAGE));
+  };
+  int t = 0;
+  for (; t < n_live; ++t) {
+    const lds_u16* kb = smem + stage * STAGE;
+    f32x16 s;
+    s_tile(kb, s);
+    copy_ahead(t);  // after this tile's S^T MFMAs: the wave waits for S anyway
+    pv_tile(kb + TILE, doc_start + t * BN, s);
+    next(t);
+  }
+  for (; t < n_tiles; ++t) {
+    copy_ahead(t);
+    next(t);
   }
 
   // O = O^T / l per query, written as whole 256-byte rows through this wave's own LDS row tile
   // (the stages are free after the last barrier); lse = (m + log2 l) ln 2.
   const float l_tot = sum_with_other_half(l_run);
   const float inv = 1.f / l_tot;
-  u32x4 w[8];  // chunk 2 db + c: d = 32 db + 16 c + 8 hi + 0..7 of query wq0 + l32
+  u32x4 w[8];  // chunk db + 4 c: d = 16 db + 64 c + 8 hi + 0..7 of query wq0 + l32
 #pragma unroll
   for (int db = 0; db < 4; ++db)
 #pragma unroll
     for (int c = 0; c < 2; ++c)
-      w[2 * db + c] = pack8<E>(oacc[db][8 * c] * inv, oacc[db][8 * c + 1] * inv,
+      w[db + 4 * c] = pack8<E>(oacc[db][8 * c] * inv, oacc[db][8 * c + 1] * inv,
                                oacc[db][8 * c + 2] * inv, oacc[db][8 * c + 3] * inv,
                                oacc[db][8 * c + 4] * inv, oacc[db][8 * c + 5] * inv,
                                oacc[db][8 * c + 6] * inv, oacc[db][8 * c + 7] * inv);
-  static_assert(NW * 32 * (8 * 16 + 8) * 2 <= 2 * STAGE * 2, "row tiles fit in LDS");
+  static_assert(NW * 32 * (8 * 16 + 8) <= NSTAGE * STAGE, "row tiles fit in LDS");
   store_rows32<16>(smem + strip * 32 * (8 * 16 + 8), w, lane,
                    [&](int r) { return o + (long)(wq0 + r) * qrow + h * D; }, q_end - wq0);
   if (q_valid && hi == 0) {
