@@ -644,6 +644,10 @@ constexpr int TILE = BN / 4 * GRP;    // halfs of a K or V tile
 constexpr int STAGE = 2 * TILE;       // K, V of one tile
 constexpr int NSTAGE = 3;
 constexpr int PER_CU = 3;             // work-groups per CU
+constexpr int64_t kThreeMinItems = 2 * PER_CU * kPlanCus;
+constexpr unsigned kPairPad = 8192;   // LDS that leaves room for two
+static_assert(PER_CU * (NSTAGE * STAGE * 2 + kPairPad) > 160 * 1024 &&
+                  2 * (NSTAGE * STAGE * 2 + kPairPad) <= 160 * 1024, "two work-groups");
 static_assert(BM / 4 * GRP <= (NSTAGE - 1) * STAGE, "the Q tile fits in stages 1 and 2");
 static_assert(PER_CU * NSTAGE * STAGE * 2 <= 160 * 1024, "LDS of three work-groups");
 static_assert(BN / 4 * 2 == 4 * NW, "copy map: 4 row groups per wave and tile pair K, V");
@@ -866,8 +870,14 @@ template <class E>
 static hipError_t launch_fwd_t(const FwdArgs& a) {
   if (a.n_items == 0) return hipSuccess;
   if (a.kernel == 2) {
-    hipLaunchKernelGGL((fwd_lean_kernel<E>), dim3((unsigned)a.n_items), dim3(fwdl::NT), 0,
-                       a.stream, (const int4*)a.items, (const uint16_t*)a.q, (const uint16_t*)a.k,
+    // Two work-groups a CU (by LDS that the kernel does not use) until the list fills the slots of
+    // three twice over (ceil(N / 128) Hq, as the kernel's own rule): in one short list each of a
+    // CU's items runs slower beside two others, and the longest sets the time. Four layers of
+    // 8192 tokens in documents of 16 to 512, 12 heads (768), captured: 460 us with three, 450 with
+    // two; 16384 tokens of 12 heads (1536): 42.3 us with three, 47.4 with two.
+    const bool three = (a.n_tokens + fwdl::BM - 1) / fwdl::BM * a.hq >= fwdl::kThreeMinItems;
+    hipLaunchKernelGGL((fwd_lean_kernel<E>), dim3((unsigned)a.n_items), dim3(fwdl::NT),
+                       three ? 0u : fwdl::kPairPad, a.stream, (const int4*)a.items, (const uint16_t*)a.q, (const uint16_t*)a.k,
                        (const uint16_t*)a.v, a.hq, a.hkv, (uint16_t*)a.out, a.lse,
                        (int)a.n_tokens, a.scale * kLog2e);
     return hipGetLastError();
