@@ -425,7 +425,7 @@ def rotary_tables(cos, sin, b_idx, t_idx):
 def rope_forward(q, k, v, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype, layout=0,
                  expand=False, batch=0, seq=0):
     """Rotated q, k and cast v as three tensors of `out_dtype`, in the packed (N, H, D) or the
-    zero-filled padded (B, H, T, D) layout; K/V keep kv_heads unless `expand`. A packed,
+    padded (B, H, T, D) layout (zeros where no token lies); K/V keep kv_heads unless `expand`. A packed,
     unexpanded v already in `out_dtype` is returned as a view of itself (the kernel leaves the
     value rows out)."""
     _require_device(q, k, v, cos, sin, b_idx, t_idx)
@@ -438,14 +438,19 @@ def rope_forward(q, k, v, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype, la
     if not (q.dtype == k.dtype == v.dtype):
         raise ValueError(f"q, k and v must share a dtype, got {q.dtype}, {k.dtype}, {v.dtype}")
     v_as_is = layout == _lib.VA_LAYOUT_PACKED and not expand and v.dtype == out_dtype
-    if layout == _lib.VA_LAYOUT_PADDED:
-        qo = torch.zeros(batch, heads, seq, HEAD_DIM, dtype=out_dtype, device=q.device)
-        ko, vo = torch.zeros_like(qo), torch.zeros_like(qo)
-    else:
-        qo = torch.empty(n, heads, HEAD_DIM, dtype=out_dtype, device=q.device)
-        ko = torch.empty(n, kvo, HEAD_DIM, dtype=out_dtype, device=q.device)
-        vo = v.view(n, kv_heads, HEAD_DIM) if v_as_is else torch.empty_like(ko)
     scb, sct = _rope_strides(cos)
+    if layout == _lib.VA_LAYOUT_PADDED:  # every row written by the kernel, zeros included
+        qo = torch.empty(batch, heads, seq, HEAD_DIM, dtype=out_dtype, device=q.device)
+        ko, vo = torch.empty_like(qo), torch.empty_like(qo)
+        row_map = torch.empty(batch * seq, dtype=torch.int32, device=q.device)
+        check(lib().va_rope_fwd_padded(
+            _ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), scb, sct, _ptr(b_idx), _ptr(t_idx),
+            _ptr(row_map), _ptr(qo), _ptr(ko), _ptr(vo), n, batch, heads, kv_heads, HEAD_DIM, seq,
+            _DTYPES[q.dtype], _DTYPES[out_dtype], _stream()), "va_rope_fwd_padded")
+        return qo, ko, vo
+    qo = torch.empty(n, heads, HEAD_DIM, dtype=out_dtype, device=q.device)
+    ko = torch.empty(n, kvo, HEAD_DIM, dtype=out_dtype, device=q.device)
+    vo = v.view(n, kv_heads, HEAD_DIM) if v_as_is else torch.empty_like(ko)
     check(lib().va_rope_fwd(_ptr(q), _ptr(k), None if v_as_is else _ptr(v), _ptr(cos), _ptr(sin),
                             scb, sct, _ptr(b_idx), _ptr(t_idx), _ptr(qo), _ptr(ko),
                             None if v_as_is else _ptr(vo), n, heads, kv_heads, HEAD_DIM, seq,
@@ -650,10 +655,11 @@ class PackRows(torch.autograd.Function):
         b_idx, t_idx = ctx.saved_tensors
         batch, heads, seq, dim = ctx.meta
         grad = grad.contiguous()
-        padded = torch.zeros(batch, heads, seq, dim, dtype=grad.dtype, device=grad.device)
-        check(lib().va_pack_rows(_ptr(grad), _ptr(padded), _ptr(b_idx), _ptr(t_idx),
-                                 b_idx.shape[0], heads, seq, dim, grad.element_size(), 1,
-                                 _stream()), "va_pack_rows")
+        padded = torch.empty(batch, heads, seq, dim, dtype=grad.dtype, device=grad.device)
+        row_map = torch.empty(batch * seq, dtype=torch.int32, device=grad.device)
+        check(lib().va_unpack_rows(_ptr(grad), _ptr(padded), _ptr(b_idx), _ptr(t_idx),
+                                   _ptr(row_map), b_idx.shape[0], batch, heads, seq, dim,
+                                   grad.element_size(), _stream()), "va_unpack_rows")
         return padded, None, None
 
 

@@ -222,6 +222,13 @@ extern "C" int va_bwd_rotary_stage(int32_t stage, const va_rope_tables* rope, co
 
 namespace {
 
+// Sizes of a padded tensor whose every row is written (row_map of batch * seq entries).
+int check_padded(int32_t batch, int32_t seq, int32_t heads, const char* what) {
+  if (batch < 0 || seq <= 0 || heads <= 0 || (int64_t)batch * seq > INT32_MAX)
+    return va::fail(VA_ESHAPE, "%s: batch=%d seq=%d heads=%d out of range", what, batch, seq, heads);
+  return VA_OK;
+}
+
 int rope_common(const void* x0, const void* x1, const void* x2, const float* cos,
                 const float* sin, const int32_t* b_idx, const int32_t* t_idx, void* y0, void* y1,
                 void* y2, int64_t n_tokens, int32_t heads, int32_t kv_heads, int32_t head_dim,
@@ -280,9 +287,35 @@ extern "C" int va_rope_fwd(const void* q, const void* k, const void* v, const fl
     return va::fail(VA_EINVAL, "va_rope_fwd: cos/sin strides must be non-negative multiples of 4");
   va::RopeArgs a{q, k, v, cos, sin, cos_batch_stride, cos_seq_stride, b_idx, t_idx,
                  q_out, k_out, v_out, n_tokens, heads, kv_heads, seq, in_dtype, out_dtype,
-                 layout, expand, (hipStream_t)stream};
+                 layout, expand, nullptr, 0, (hipStream_t)stream};
   hipError_t e = va::launch_rope_fwd(a);
   return e == hipSuccess ? VA_OK : hip_fail(e, "va_rope_fwd launch");
+}
+
+extern "C" int va_rope_fwd_padded(const void* q, const void* k, const void* v, const float* cos,
+                                  const float* sin, int64_t cos_batch_stride,
+                                  int64_t cos_seq_stride, const int32_t* b_idx,
+                                  const int32_t* t_idx, int32_t* row_map, void* q_out, void* k_out,
+                                  void* v_out, int64_t n_tokens, int32_t batch, int32_t heads,
+                                  int32_t kv_heads, int32_t head_dim, int32_t seq,
+                                  int32_t in_dtype, int32_t out_dtype, void* stream) {
+  int rc = rope_common(q, k, v, cos, sin, b_idx, t_idx, q_out, k_out, v_out, n_tokens, heads,
+                       kv_heads, head_dim, seq, in_dtype, out_dtype, VA_LAYOUT_PADDED, 1,
+                       "va_rope_fwd_padded");
+  if (rc) return rc;
+  if ((rc = check_padded(batch, seq, heads, "va_rope_fwd_padded"))) return rc;
+  if (batch == 0) return VA_OK;
+  if ((rc = check_ptrs({row_map, q_out, k_out, v_out}, "va_rope_fwd_padded"))) return rc;
+  if (cos_batch_stride % 4 != 0 || cos_seq_stride % 4 != 0 || cos_batch_stride < 0 ||
+      cos_seq_stride < 0)
+    return va::fail(VA_EINVAL,
+                    "va_rope_fwd_padded: cos/sin strides must be non-negative multiples of 4");
+  va::RopeArgs a{q, k, v, cos, sin, cos_batch_stride, cos_seq_stride, b_idx, t_idx,
+                 q_out, k_out, v_out, n_tokens, heads, kv_heads, seq, in_dtype, out_dtype,
+                 VA_LAYOUT_PADDED, 1, row_map, batch, (hipStream_t)stream};
+  hipError_t e = va::launch_row_map(b_idx, t_idx, n_tokens, batch, seq, row_map, a.stream);
+  if (e == hipSuccess) e = va::launch_rope_fwd(a);
+  return e == hipSuccess ? VA_OK : hip_fail(e, "va_rope_fwd_padded launch");
 }
 
 extern "C" int va_rope_bwd(const void* dq, const void* dk, const void* dv, const float* cos,
@@ -300,7 +333,7 @@ extern "C" int va_rope_bwd(const void* dq, const void* dk, const void* dv, const
     return va::fail(VA_EINVAL, "va_rope_bwd: cos/sin strides must be non-negative multiples of 4");
   va::RopeArgs a{dq, dk, dv, cos, sin, cos_batch_stride, cos_seq_stride, b_idx, t_idx,
                  dq_in, dk_in, dv_in, n_tokens, heads, kv_heads, seq, in_dtype, out_dtype,
-                 layout, expand, (hipStream_t)stream};
+                 layout, expand, nullptr, 0, (hipStream_t)stream};
   hipError_t e = va::launch_rope_bwd(a);
   return e == hipSuccess ? VA_OK : hip_fail(e, "va_rope_bwd launch");
 }
@@ -322,4 +355,27 @@ extern "C" int va_pack_rows(const void* src, void* dst, const int32_t* b_idx,
   hipError_t e = va::launch_pack_rows(src, dst, b_idx, t_idx, n_tokens, heads, seq,
                                       (int)row_bytes, mode, (hipStream_t)stream);
   return e == hipSuccess ? VA_OK : hip_fail(e, "va_pack_rows launch");
+}
+
+extern "C" int va_unpack_rows(const void* src, void* dst, const int32_t* b_idx,
+                              const int32_t* t_idx, int32_t* row_map, int64_t n_tokens,
+                              int32_t batch, int32_t heads, int32_t seq, int32_t head_dim,
+                              int32_t elem_bytes, void* stream) {
+  if (elem_bytes != 2 && elem_bytes != 4) return va::fail(VA_EDTYPE, "va_unpack_rows: elem_bytes");
+  if (head_dim <= 0 || n_tokens < 0 || n_tokens > INT32_MAX || heads > 65535)
+    return va::fail(VA_ESHAPE, "va_unpack_rows: sizes");
+  int rc = check_padded(batch, seq, heads, "va_unpack_rows");
+  if (rc) return rc;
+  const int64_t row_bytes = (int64_t)head_dim * elem_bytes;
+  if (row_bytes % 16 != 0 || row_bytes / 16 > 1024)
+    return va::fail(VA_ESHAPE, "va_unpack_rows: head_dim * elem_bytes must be a multiple of 16");
+  if (batch == 0) return VA_OK;
+  if (n_tokens > 0 && (rc = check_ptrs({src, b_idx, t_idx}, "va_unpack_rows"))) return rc;
+  if ((rc = check_ptrs({dst, row_map}, "va_unpack_rows"))) return rc;
+  hipError_t e = va::launch_row_map(b_idx, t_idx, n_tokens, batch, seq, row_map,
+                                    (hipStream_t)stream);
+  if (e == hipSuccess)
+    e = va::launch_unpack_rows(src, dst, row_map, b_idx, t_idx, n_tokens, batch, heads, seq,
+                               (int)row_bytes, (hipStream_t)stream);
+  return e == hipSuccess ? VA_OK : hip_fail(e, "va_unpack_rows launch");
 }

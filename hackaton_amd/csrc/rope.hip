@@ -8,7 +8,9 @@
 // rope_bwd_kernel   the inverse rotation of dq and dk and the cast of dv, after summing the G
 //                   copies (or per-head partials) of dk/dv in fp32 when they are per query head;
 //                   output in the projection type.
+// row_map_kernel    the inverse of (b_idx, t_idx): which token, if any, a padded row holds.
 // pack_rows_kernel  (B, H, T, D) <-> (N, H*D) gather / scatter of whole 16-byte chunks.
+// unpack_rows_kernel  the scatter over a row map: every padded row written once, zeros included.
 //
 // Access pattern: one wave per token. A (token, head) row of D = 128 elements is handled by 8
 // consecutive lanes; lane j of the row takes elements [8j, 8j + 8) of the first half and the
@@ -201,18 +203,32 @@ __device__ inline void fwd_store(const RopeArgs& a, long pid, int b, int t, int 
   }
 }
 
+// row_map[b * seq + t] = the token at (b, t). Rows without a token keep whatever the caller's
+// memory holds: a reader takes an entry only if it names a token that lies at that row
+// (token_at), so the map needs no clearing.
+__global__ void row_map_kernel(const int32_t* __restrict__ b_idx,
+                               const int32_t* __restrict__ t_idx, int32_t* __restrict__ row_map,
+                               int n_tokens, int batch, int seq) {
+  const int pid = blockIdx.x * blockDim.x + threadIdx.x;
+  if (pid >= n_tokens) return;
+  const int b = b_idx[pid], t = t_idx[pid];
+  if (b >= 0 && b < batch && t >= 0 && t < seq) row_map[(long)b * seq + t] = pid;
+}
+__device__ inline int token_at(const int32_t* row_map, const int32_t* b_idx, const int32_t* t_idx,
+                               int n_tokens, long row, int b, int t) {
+  const int pid = row_map[row];
+  if (pid < 0 || pid >= n_tokens) return -1;
+  return b_idx[pid] == b && t_idx[pid] == t ? pid : -1;
+}
+
 // Each lane group handles two rows per pass: both rows, then the token's cos / sin chunks, are
 // loaded before either row is stored, so a wave has the reads of 16 rows in flight (all 16 rows
 // of a 12 + 2 + 2 head token in one pass). The tables are read again per pass, from cache.
 template <int IN, int OUT>
-__global__ __launch_bounds__(kRopeThreads) void rope_fwd_kernel(RopeArgs a) {
-  const TokenLanes tl = token_lanes(a.n_tokens);
-  if (!tl.valid) return;
-  const long pid = tl.pid;
-  const int c0 = 8 * tl.j;
-  const int b = a.b_idx[pid], t = a.t_idx[pid];
+__device__ inline void fwd_token(const RopeArgs& a, long pid, int b, int t) {
+  const int c0 = 8 * (threadIdx.x & 7);
   const int slots = a.heads + (a.x2 != nullptr ? 2 : 1) * a.kv_heads;  // no value rows: x2 null
-  for (int s0 = tl.r0; s0 < slots; s0 += 16) {
+  for (int s0 = (threadIdx.x & 63) >> 3; s0 < slots; s0 += 16) {
     const int s1 = s0 + 8;
     const RowIn<IN> u = fwd_load<IN>(a, pid, c0, s0);
     RowIn<IN> w;
@@ -221,6 +237,38 @@ __global__ __launch_bounds__(kRopeThreads) void rope_fwd_kernel(RopeArgs a) {
     load_tables(a, b, t, c0, tb);
     fwd_store<IN, OUT>(a, pid, b, t, c0, s0, tb, u);
     if (s1 < slots) fwd_store<IN, OUT>(a, pid, b, t, c0, s1, tb, w);
+  }
+}
+
+template <int IN, int OUT>
+__global__ __launch_bounds__(kRopeThreads) void rope_fwd_kernel(RopeArgs a) {
+  const TokenLanes tl = token_lanes(a.n_tokens);
+  if (!tl.valid) return;
+  fwd_token<IN, OUT>(a, tl.pid, a.b_idx[tl.pid], a.t_idx[tl.pid]);
+}
+
+// The padded layout, every row written once: one wave per padded row (b, t), which holds a token
+// (rotated as above) or zeros. Writing the rows of a zero-filled tensor instead moved the real
+// rows' bytes twice: at 34 rows of 1024 with 18,432 tokens, 12 / 2 heads, fp16, the fills (three
+// 107 MB tensors) and the rotation took 92 us, the row map and this kernel 81 us (396 MB, 4.9 TB/s).
+template <int IN, int OUT>
+__global__ __launch_bounds__(kRopeThreads) void rope_fwd_padded_kernel(RopeArgs a) {
+  const long row =
+      (long)blockIdx.x * kTokensPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (row >= (long)a.batch * a.seq) return;
+  const int b = (int)(row / a.seq), t = (int)(row - (long)b * a.seq);
+  const int pid = token_at(a.row_map, a.b_idx, a.t_idx, (int)a.n_tokens, row, b, t);
+  if (pid >= 0) {
+    fwd_token<IN, OUT>(a, pid, b, t);
+    return;
+  }
+  constexpr int kChunks = D * (OUT == kF32 ? 4 : 2) / 16;
+  for (int i = threadIdx.x & 63; i < a.heads * kChunks; i += 64) {
+    const int head = i / kChunks, c = i % kChunks;
+    const long at = (((long)b * a.heads + head) * a.seq + t) * kChunks + c;
+    reinterpret_cast<u32x4*>(a.y0)[at] = u32x4{0u, 0u, 0u, 0u};
+    reinterpret_cast<u32x4*>(a.y1)[at] = u32x4{0u, 0u, 0u, 0u};
+    reinterpret_cast<u32x4*>(a.y2)[at] = u32x4{0u, 0u, 0u, 0u};
   }
 }
 
@@ -249,7 +297,8 @@ __device__ inline void bwd_store(const RopeArgs& a, long pid, int b, int t, int 
   cvt8<IN>(in.h2, d2);
   const int copies = (!sl.is_q && a.expand) ? a.heads / a.kv_heads : 1;
   // The other copies in batches of 7, every load of a batch issued before its first add: one
-  // memory round trip per batch instead of one per copy.
+  // memory round trip per batch instead of one per copy. (Loading the first batch beside the other
+  // rows of the pass takes 205 registers: 47.5 -> 53 us at 18,432 tokens of 12 / 2 heads, fp16.)
   constexpr int kBatch = 7;
   for (int r0 = 1; r0 < copies; r0 += kBatch) {
     RowIn<IN> more[kBatch];
@@ -303,25 +352,91 @@ __global__ __launch_bounds__(kRopeThreads) void rope_bwd_kernel(RopeArgs a) {
   }
 }
 
-// grid (N, heads) x (row_chunks) threads; 16-byte chunks of one (token, head) row.
-__global__ void pack_rows_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst,
-                                 const int32_t* __restrict__ b_idx,
-                                 const int32_t* __restrict__ t_idx, int heads, int seq,
-                                 int row_chunks, int mode) {
-  const long pid = blockIdx.x;
-  const int head = blockIdx.y;
-  const int c = threadIdx.x;
-  if (c >= row_chunks) return;
-  const long padded = (((long)b_idx[pid] * heads + head) * seq + t_idx[pid]) * row_chunks + c;
-  const long packed = (pid * heads + head) * row_chunks + c;
-  if (mode == 0) dst[packed] = src[padded];
-  else dst[padded] = src[packed];
+// --------------------------------------------------------------------------------------------
+// Row packing: one wave per token (or padded row), which walks the heads * row_chunks 16-byte
+// chunks of the token's packed row, 4 loads in flight per lane; row_chunks a power of two (2^LOG)
+// or any number (LOG < 0). Bound by HBM: the gather of 18,432 tokens of 12 heads, fp16 (113 MB):
+// 50 us with a 16-thread work-group per (token, head), 18 us (6.2 TB/s, part of it from the
+// last-level cache) with a wave per token. The scatter into 34 rows of 1024 (107 MB written):
+// 65 us with a fill and that kernel, 26 us with the row map and every row written once.
+// --------------------------------------------------------------------------------------------
+template <int LOG>
+struct Chunk {
+  int head, c;
+  __device__ Chunk(int i, int row_chunks) {
+    head = LOG >= 0 ? i >> (LOG < 0 ? 0 : LOG) : i / row_chunks;
+    c = LOG >= 0 ? i & ((1 << (LOG < 0 ? 0 : LOG)) - 1) : i - head * row_chunks;
+  }
+};
+constexpr int kPackThreads = 256, kPackWaves = kPackThreads / 64, kPackLoads = 4;
+
+template <int LOG>
+__global__ __launch_bounds__(kPackThreads) void pack_rows_kernel(
+    const u32x4* __restrict__ src, u32x4* __restrict__ dst, const int32_t* __restrict__ b_idx,
+    const int32_t* __restrict__ t_idx, long n_tokens, int heads, int seq, int row_chunks,
+    int mode) {
+  const long pid =
+      (long)blockIdx.x * kPackWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (pid >= n_tokens) return;
+  const int total = heads * row_chunks;
+  const long padded0 = (long)b_idx[pid] * heads * seq + t_idx[pid];
+  for (int i0 = threadIdx.x & 63; i0 < total; i0 += 64 * kPackLoads) {
+    u32x4 w[kPackLoads];
+#pragma unroll
+    for (int j = 0; j < kPackLoads; ++j) {
+      const int i = i0 + 64 * j;
+      const Chunk<LOG> ch(i, row_chunks);
+      const long padded = (padded0 + (long)ch.head * seq) * row_chunks + ch.c;
+      if (i < total) w[j] = src[mode == 0 ? padded : pid * total + i];
+    }
+#pragma unroll
+    for (int j = 0; j < kPackLoads; ++j) {
+      const int i = i0 + 64 * j;
+      const Chunk<LOG> ch(i, row_chunks);
+      const long padded = (padded0 + (long)ch.head * seq) * row_chunks + ch.c;
+      if (i < total) dst[mode == 0 ? pid * total + i : padded] = w[j];
+    }
+  }
+}
+
+template <int LOG>
+__global__ __launch_bounds__(kPackThreads) void unpack_rows_kernel(
+    const u32x4* __restrict__ src, u32x4* __restrict__ dst, const int32_t* __restrict__ row_map,
+    const int32_t* __restrict__ b_idx, const int32_t* __restrict__ t_idx, int n_tokens, long rows,
+    int heads, int seq, int row_chunks) {
+  const long row =
+      (long)blockIdx.x * kPackWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int b = (int)(row / seq), t = (int)(row - (long)b * seq);
+  const int pid = token_at(row_map, b_idx, t_idx, n_tokens, row, b, t);
+  const int total = heads * row_chunks;
+  const long padded0 = (long)b * heads * seq + t;
+  for (int i0 = threadIdx.x & 63; i0 < total; i0 += 64 * kPackLoads) {
+    u32x4 w[kPackLoads];
+#pragma unroll
+    for (int j = 0; j < kPackLoads; ++j) {
+      const int i = i0 + 64 * j;
+      w[j] = u32x4{0u, 0u, 0u, 0u};
+      if (pid >= 0 && i < total) w[j] = src[(long)pid * total + i];
+    }
+#pragma unroll
+    for (int j = 0; j < kPackLoads; ++j) {
+      const int i = i0 + 64 * j;
+      const Chunk<LOG> ch(i, row_chunks);
+      if (i < total) dst[(padded0 + (long)ch.head * seq) * row_chunks + ch.c] = w[j];
+    }
+  }
 }
 
 template <int IN, int OUT>
 hipError_t launch_rope_t(const RopeArgs& a, bool fwd) {
   const unsigned groups = (unsigned)((a.n_tokens + kTokensPerGroup - 1) / kTokensPerGroup);
-  if (fwd) {
+  if (fwd && a.row_map != nullptr) {
+    const long rows = (long)a.batch * a.seq;
+    hipLaunchKernelGGL((rope_fwd_padded_kernel<IN, OUT>),
+                       dim3((unsigned)((rows + kTokensPerGroup - 1) / kTokensPerGroup)),
+                       dim3(kRopeThreads), 0, a.stream, a);
+  } else if (fwd) {
     hipLaunchKernelGGL((rope_fwd_kernel<IN, OUT>), dim3(groups), dim3(kRopeThreads), 0, a.stream,
                        a);
   } else {
@@ -341,7 +456,7 @@ hipError_t launch_rope_out(const RopeArgs& a, bool fwd) {
 }
 
 hipError_t launch_rope(const RopeArgs& a, bool fwd) {
-  if (a.n_tokens == 0) return hipSuccess;
+  if (a.row_map != nullptr ? (long)a.batch * a.seq == 0 : a.n_tokens == 0) return hipSuccess;
   switch (a.in_dtype) {
     case kF16: return launch_rope_out<kF16>(a, fwd);
     case kBF16: return launch_rope_out<kBF16>(a, fwd);
@@ -359,8 +474,35 @@ hipError_t launch_pack_rows(const void* src, void* dst, const int32_t* b_idx, co
                             hipStream_t stream) {
   if (n_tokens == 0) return hipSuccess;
   const int chunks = row_bytes / 16;
-  hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)n_tokens, heads), dim3(chunks), 0, stream,
-                     (const u32x4*)src, (u32x4*)dst, b_idx, t_idx, heads, seq, chunks, mode);
+  const dim3 grid((unsigned)((n_tokens + kPackWaves - 1) / kPackWaves));
+  const auto kernel = chunks == 16   ? pack_rows_kernel<4>
+                      : chunks == 32 ? pack_rows_kernel<5>
+                                     : pack_rows_kernel<-1>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kPackThreads), 0, stream, (const u32x4*)src, (u32x4*)dst,
+                     b_idx, t_idx, (long)n_tokens, heads, seq, chunks, mode);
+  return hipGetLastError();
+}
+
+hipError_t launch_row_map(const int32_t* b_idx, const int32_t* t_idx, int64_t n_tokens, int batch,
+                          int seq, int32_t* row_map, hipStream_t stream) {
+  if (n_tokens == 0) return hipSuccess;
+  hipLaunchKernelGGL(row_map_kernel, dim3((unsigned)((n_tokens + 255) / 256)), dim3(256), 0, stream,
+                     b_idx, t_idx, row_map, (int)n_tokens, batch, seq);
+  return hipGetLastError();
+}
+
+hipError_t launch_unpack_rows(const void* src, void* dst, const int32_t* row_map,
+                              const int32_t* b_idx, const int32_t* t_idx, int64_t n_tokens,
+                              int batch, int heads, int seq, int row_bytes, hipStream_t stream) {
+  const long rows = (long)batch * seq;
+  if (rows == 0) return hipSuccess;
+  const int chunks = row_bytes / 16;
+  const dim3 grid((unsigned)((rows + kPackWaves - 1) / kPackWaves));
+  const auto kernel = chunks == 16   ? unpack_rows_kernel<4>
+                      : chunks == 32 ? unpack_rows_kernel<5>
+                                     : unpack_rows_kernel<-1>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kPackThreads), 0, stream, (const u32x4*)src, (u32x4*)dst,
+                     row_map, b_idx, t_idx, (int)n_tokens, rows, heads, seq, chunks);
   return hipGetLastError();
 }
 

@@ -141,6 +141,8 @@ struct RopeArgs {
   int out_dtype;         // dtype of y
   int layout;            // 0 packed (N, H, D); 1 padded (B, H, T, D)
   int expand;            // 1: write K/V for every query head (reference qkv_rotate semantics)
+  const int32_t* row_map;  // padded forward that writes every row: (batch * seq), else null
+  int batch;
   hipStream_t stream;
 };
 
@@ -153,6 +155,13 @@ hipError_t launch_rope_bwd(const RopeArgs& a);
 hipError_t launch_pack_rows(const void* src, void* dst, const int32_t* b_idx, const int32_t* t_idx,
                             int64_t n_tokens, int heads, int seq, int row_bytes, int mode,
                             hipStream_t stream);
+// row_map (batch * seq) from the tokens' positions; the scatter over it (padded rows without a
+// token become zeros).
+hipError_t launch_row_map(const int32_t* b_idx, const int32_t* t_idx, int64_t n_tokens, int batch,
+                          int seq, int32_t* row_map, hipStream_t stream);
+hipError_t launch_unpack_rows(const void* src, void* dst, const int32_t* row_map,
+                              const int32_t* b_idx, const int32_t* t_idx, int64_t n_tokens,
+                              int batch, int heads, int seq, int row_bytes, hipStream_t stream);
 
 // Device-built plans (plan_device.hip): from a device cu_seqlens or from device lengths (exactly
 // one non-null); each requested plan (non-null items) is `capacity` items, real ones first, empty

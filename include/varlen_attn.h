@@ -248,6 +248,10 @@ int va_bwd_rotary_stage(int32_t stage, const va_rope_tables* rope, const void* d
  * (reference qkv_rotate semantics); expand=0 keeps kv_heads (GQA-native attention input).
  * v and v_out may both be NULL in a forward without expand: only the q and k rows are written
  * (for a caller whose v is already in out_dtype and uses it as it is).
+ * va_rope_fwd_padded is the forward in the padded layout (expand = 1) for outputs that hold
+ * anything: it writes every row of (batch, heads, seq, D), zeros where no token lies. row_map is
+ * scratch of batch * seq int32, 16-byte aligned, whose contents do not matter; tokens outside
+ * (batch, seq) are left out.
  * Backward: the inverse rotation (and the sum of the G copies when expand=1); dq/dk/dv read in
  * in_dtype from `layout`, written (N, H*D) in out_dtype. Every tensor base must be 16-byte aligned
  * and the cos/sin strides (in elements) non-negative multiples of 4: each lane moves 16 bytes.
@@ -257,6 +261,12 @@ int va_rope_fwd(const void* q, const void* k, const void* v, const float* cos, c
                 const int32_t* t_idx, void* q_out, void* k_out, void* v_out, int64_t n_tokens,
                 int32_t heads, int32_t kv_heads, int32_t head_dim, int32_t seq, int32_t in_dtype,
                 int32_t out_dtype, int32_t layout, int32_t expand, void* stream);
+int va_rope_fwd_padded(const void* q, const void* k, const void* v, const float* cos,
+                       const float* sin, int64_t cos_batch_stride, int64_t cos_seq_stride,
+                       const int32_t* b_idx, const int32_t* t_idx, int32_t* row_map, void* q_out,
+                       void* k_out, void* v_out, int64_t n_tokens, int32_t batch, int32_t heads,
+                       int32_t kv_heads, int32_t head_dim, int32_t seq, int32_t in_dtype,
+                       int32_t out_dtype, void* stream);
 int va_rope_bwd(const void* dq, const void* dk, const void* dv, const float* cos,
                 const float* sin, int64_t cos_batch_stride, int64_t cos_seq_stride,
                 const int32_t* b_idx, const int32_t* t_idx, void* dq_in, void* dk_in,
@@ -267,10 +277,15 @@ int va_rope_bwd(const void* dq, const void* dk, const void* dv, const float* cos
 /* ---- row packing ------------------------------------------------------------------------------
  * mode 0: (B, heads, seq, head_dim) -> (N, heads*head_dim) rows of the real tokens (exact);
  * mode 1: the reverse scatter into a caller-zeroed (B, heads, seq, head_dim) buffer.
+ * va_unpack_rows is the scatter into a buffer that holds anything: every row of (batch, heads,
+ * seq, head_dim) is written, zeros where no token lies (row_map: scratch as in va_rope_fwd_padded).
  * Replaces: solution/attention.py:288-300 (pack_kernel). */
 int va_pack_rows(const void* src, void* dst, const int32_t* b_idx, const int32_t* t_idx,
                  int64_t n_tokens, int32_t heads, int32_t seq, int32_t head_dim,
                  int32_t elem_bytes, int32_t mode, void* stream);
+int va_unpack_rows(const void* src, void* dst, const int32_t* b_idx, const int32_t* t_idx,
+                   int32_t* row_map, int64_t n_tokens, int32_t batch, int32_t heads, int32_t seq,
+                   int32_t head_dim, int32_t elem_bytes, void* stream);
 
 /* ---- machine-ceiling probes (diagnostics) ----------------------------------------------------
  * No counterpart in the reference: the benchmark measures with them the two ceilings it quotes
