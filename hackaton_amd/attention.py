@@ -25,6 +25,7 @@ Every op requires the HIP library and CUDA (HIP) tensors; there is no other impl
 """
 
 import ctypes
+import functools
 
 import numpy as np
 import torch
@@ -39,11 +40,9 @@ _DTYPES = {torch.float16: _lib.VA_F16, torch.bfloat16: _lib.VA_BF16, torch.float
 
 
 def _stream():
-    return ctypes_stream(torch.cuda.current_stream())
-
-
-def ctypes_stream(stream):
-    return stream.cuda_stream
+    """The current device's current stream as an integer: torch.cuda.current_stream().cuda_stream
+    without the Stream object, which costs as much as a launch."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
@@ -84,6 +83,7 @@ def _cu_seqlens(lengths, device):
             offsets.append(offsets[-1] + int(length))
         cu = torch.tensor(offsets, dtype=torch.int32, device=device)
         cu._va_offsets = tuple(offsets)
+        cu._va_host_plans = {}  # (Hq, Hkv) -> Plan, beside the offsets that they are made from
         _CU_SEQLENS[key] = cu
     return cu
 
@@ -159,6 +159,15 @@ def build_plan_host(cu, hq, hkv, kind):
     return items[: int(n[0])]
 
 
+@functools.lru_cache(maxsize=64)
+def _plan_capacity(n_tokens, n_docs, hq, kind):
+    """Items of a device-built plan for these sizes."""
+    cap = ctypes.c_int64()
+    check(lib().va_plan_capacity(n_tokens, n_docs, hq, kind, ctypes.byref(cap)),
+          "va_plan_capacity")
+    return cap.value
+
+
 class DevicePlan:
     """Work lists and cu_seqlens built on the device from device lengths: no host read. One launch
     (va_plan_build_device_lengths) builds cu_seqlens, the forward list (VA_PLAN_FWD_NARROW, as the
@@ -179,13 +188,8 @@ class DevicePlan:
         n_docs = lengths.numel()
         self.total = int(n_tokens)
         dev = lengths.device
-        caps = []
-        for kind in (_lib.VA_PLAN_FWD_NARROW, _lib.VA_PLAN_BWD):
-            cap = np.zeros(1, dtype=np.int64)
-            check(lib().va_plan_capacity(n_tokens, n_docs, hq, kind, cap.ctypes.data_as(_lib._pi64)),
-                  "va_plan_capacity")
-            caps.append(int(cap[0]))
-        self.n_fwd, self.n_bwd = caps
+        self.n_fwd = _plan_capacity(self.total, n_docs, hq, _lib.VA_PLAN_FWD_NARROW)
+        self.n_bwd = _plan_capacity(self.total, n_docs, hq, _lib.VA_PLAN_BWD)
         self.fwd_items = torch.empty(max(self.n_fwd, 1), 4, dtype=torch.int32, device=dev)
         part = torch.empty(max(self.n_bwd, 1), 4, dtype=torch.int32, device=dev)
         self.cu = torch.empty(n_docs + 1, dtype=torch.int32, device=dev)
@@ -236,12 +240,17 @@ def _device_plan(lengths, n_tokens, hq, hkv):
 
 
 def _plan(cu_seqlens, hq, hkv):
+    known = getattr(cu_seqlens, "_va_host_plans", None)
+    if known is not None:
+        plan = known.get((hq, hkv))
+        if plan is None:
+            plan = known[(hq, hkv)] = Plan(cu_seqlens._va_offsets, hq, hkv, cu_seqlens.device)
+        return plan
     device_plan = getattr(cu_seqlens, "_va_plan", None)
     if device_plan is not None:
         return device_plan
-    offsets = getattr(cu_seqlens, "_va_offsets", None)
-    if offsets is None:  # a cu_seqlens tensor not made by _cu_seqlens: read it (one sync)
-        offsets = tuple(int(x) for x in cu_seqlens.cpu().tolist())
+    # a cu_seqlens tensor not made by _cu_seqlens: read it (one sync)
+    offsets = tuple(int(x) for x in cu_seqlens.cpu().tolist())
     key = (cu_seqlens.device, offsets, hq, hkv)
     plan = _PLANS.get(key)
     if plan is None:
@@ -259,20 +268,21 @@ def attention_forward(query, key, value, plan, scale):
     key/value (N, Hkv, D), all contiguous, same 16-bit dtype."""
     _require_device(query, key, value)
     dtype = _attn_dtype(query)
-    if key.dtype != query.dtype or value.dtype != query.dtype:
+    if not (key.dtype == value.dtype == query.dtype):
         raise ValueError("query, key and value must share a dtype")
     n, hq, d = query.shape
-    hkv = key.shape[1]
-    if key.shape != (n, hkv, d) or value.shape != key.shape:
+    k_shape = key.shape
+    hkv = k_shape[1]
+    if k_shape != (n, hkv, d) or value.shape != k_shape:
         raise ValueError(f"shape mismatch: q {tuple(query.shape)} k {tuple(key.shape)} "
                          f"v {tuple(value.shape)}")
     if n != plan.total:
         raise ValueError(f"{n} tokens but cu_seqlens covers {plan.total}")
     out = torch.empty_like(query)
     lse = torch.empty(hq, n, dtype=torch.float32, device=query.device)
-    check(lib().va_fwd(_ptr(query), _ptr(key), _ptr(value), _ptr(out), _ptr(lse),
-                       _ptr(plan.fwd_items), plan.n_fwd, n, hq, hkv, d, float(scale), dtype,
-                       _stream()), "va_fwd")
+    check(lib().va_fwd(query.data_ptr(), key.data_ptr(), value.data_ptr(), out.data_ptr(),
+                       lse.data_ptr(), plan.fwd_items.data_ptr(), plan.n_fwd, n, hq, hkv, d,
+                       float(scale), dtype, _stream()), "va_fwd")
     return out, lse
 
 
@@ -283,15 +293,21 @@ def bwd_workspace_needed(hq, hkv, outputs=True):
     return hq != hkv or not outputs
 
 
+@functools.lru_cache(maxsize=64)
+def _workspace_layout(n, hq, hkv):
+    """(bytes, byte offsets of the two partial arrays) of the backward's workspace."""
+    offsets = (ctypes.c_int64 * 2)()
+    nbytes = ctypes.c_int64()
+    check(lib().va_bwd_workspace_layout(n, hq, hkv, HEAD_DIM, offsets, ctypes.byref(nbytes)),
+          "va_bwd_workspace_layout")
+    return nbytes.value, tuple(offsets)
+
+
 def bwd_workspace(n, hq, hkv, device):
     """Workspace of the backward (per-query-head dK/dV partials, row flags, row statistics) and
     the byte offsets of the two partial arrays."""
-    offsets = np.zeros(2, dtype=np.int64)
-    nbytes = np.zeros(1, dtype=np.int64)
-    check(lib().va_bwd_workspace_layout(n, hq, hkv, HEAD_DIM, offsets.ctypes.data_as(_lib._pi64),
-                                        nbytes.ctypes.data_as(_lib._pi64)),
-          "va_bwd_workspace_layout")
-    return torch.empty(int(nbytes[0]), dtype=torch.uint8, device=device), [int(x) for x in offsets]
+    nbytes, offsets = _workspace_layout(n, hq, hkv)
+    return torch.empty(nbytes, dtype=torch.uint8, device=device), list(offsets)
 
 
 def bwd_stages(plan, outputs=True, workspace=True):
@@ -311,13 +327,29 @@ def attention_backward(grad, query, key, value, out, lse, plan, scale, outputs=T
     type (plus the workspace that holds them), for a caller that sums them itself. With `rope`
     (rotary_tables(...)) dq and dk come out rotated back to the projections' frame by the
     kernels' epilogues (va_bwd_rotary_stage)."""
+    dq, dk, dv, ws, offs = _attention_backward(grad, query, key, value, out, lse, plan, scale,
+                                               outputs, rope)
+    if outputs:
+        return dq, dk, dv
+    part = query.numel() * 2
+
+    def view(off):
+        return ws[off: off + part].view(query.dtype).view(query.shape)
+
+    return dq, view(offs[0]), view(offs[1]), ws
+
+
+def _attention_backward(grad, query, key, value, out, lse, plan, scale, outputs, rope=None):
+    """(dq, dk, dv, workspace, byte offsets of the dK and dV partials in it): dk and dv are None
+    without outputs, workspace and offsets where there is none."""
     n, hq, d = query.shape
     hkv = key.shape[1]
     dtype = _attn_dtype(query)
-    grad = grad.reshape(out.shape)
+    if grad.numel() != out.numel():
+        raise RuntimeError(f"gradient of {tuple(grad.shape)} for an output of {tuple(out.shape)}")
     if grad.dtype != query.dtype:
         grad = grad.to(query.dtype)
-    grad = grad.contiguous()
+    grad = grad.contiguous()  # (N, Hq * D) or (N, Hq, D): the same rows
     dq = torch.empty_like(query)
     if outputs:
         dk, dv = torch.empty_like(key), torch.empty_like(value)
@@ -338,14 +370,7 @@ def attention_backward(grad, query, key, value, out, lse, plan, scale, outputs=T
         else:
             check(lib().va_bwd_rotary_stage(stage, ctypes.byref(rope[0]), *argv),
                   "va_bwd_rotary_stage")
-    if outputs:
-        return dq, dk, dv
-    part = n * hq * d * 2
-
-    def view(off):
-        return ws[off: off + part].view(query.dtype).view(n, hq, d)
-
-    return dq, view(offs[0]), view(offs[1]), ws
+    return dq, dk, dv, ws, offs
 
 
 class VarlenAttention(torch.autograd.Function):
@@ -375,7 +400,7 @@ def _lengths_cu(lengths, device, hq, hkv, n_tokens):
     built on the device by one launch, cached on the tensor: no host read, no synchronisation)."""
     if isinstance(lengths, torch.Tensor) and lengths.is_cuda:
         return _device_plan(lengths, n_tokens, hq, hkv).cu, None
-    lengths = [int(length) for length in lengths if int(length) > 0]
+    lengths = [length for length in map(int, lengths) if length > 0]
     if not lengths:  # the reference's max() of no lengths raises ValueError too (attention.py:242)
         raise ValueError("varlen attention: every length is zero (no tokens to attend over)")
     return _cu_seqlens(lengths, device), max(lengths)
@@ -397,14 +422,17 @@ def varlen_attention(query, key, value, lengths, scale):
 # rotary embedding
 # ------------------------------------------------------------------------------------------------
 def _rope_strides(cos):
-    scb = 0 if cos.shape[0] == 1 else cos.stride(0)
-    return scb, cos.stride(1)
+    strides = cos.stride()
+    return 0 if cos.shape[0] == 1 else strides[0], strides[1]
 
 
 def _tables(cos, sin):
-    cos = cos.float().contiguous()
-    sin = sin.float().contiguous()
-    if cos.shape != sin.shape or cos.dim() != 3 or cos.shape[-1] != HEAD_DIM:
+    if cos.dtype != torch.float32 or not cos.is_contiguous():
+        cos = cos.float().contiguous()
+    if sin.dtype != torch.float32 or not sin.is_contiguous():
+        sin = sin.float().contiguous()
+    shape = cos.shape
+    if sin.shape != shape or len(shape) != 3 or shape[2] != HEAD_DIM:
         raise ValueError(f"cos/sin must be (1 or B, T, {HEAD_DIM}), got {tuple(cos.shape)}")
     return cos, sin
 
@@ -425,15 +453,16 @@ def rotary_tables(cos, sin, b_idx, t_idx):
 def rope_forward(q, k, v, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype, layout=0,
                  expand=False, batch=0, seq=0):
     """Rotated q, k and cast v as three tensors of `out_dtype`, in the packed (N, H, D) or the
-    padded (B, H, T, D) layout (zeros where no token lies); K/V keep kv_heads unless `expand`. A packed,
-    unexpanded v already in `out_dtype` is returned as a view of itself (the kernel leaves the
-    value rows out)."""
+    padded (B, H, T, D) layout (zeros where no token lies); K/V keep kv_heads unless `expand`. A
+    packed, unexpanded v already in `out_dtype` is returned as a view of itself (the kernel leaves
+    the value rows out)."""
     _require_device(q, k, v, cos, sin, b_idx, t_idx)
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     cos, sin = _tables(cos, sin)
     n = q.shape[0]
     kvo = heads if expand else kv_heads
-    if q.shape[1] != heads * HEAD_DIM or k.shape[1] != kv_heads * HEAD_DIM or v.shape != k.shape:
+    k_shape = k.shape
+    if q.shape[1] != heads * HEAD_DIM or k_shape[1] != kv_heads * HEAD_DIM or v.shape != k_shape:
         raise ValueError("projection shapes do not match heads * head_dim")
     if not (q.dtype == k.dtype == v.dtype):
         raise ValueError(f"q, k and v must share a dtype, got {q.dtype}, {k.dtype}, {v.dtype}")
@@ -463,19 +492,26 @@ def rope_backward(dq, dk, dv, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype
                   expand=False, seq=0):
     """Projection gradients (N, heads*D), (N, kv_heads*D) x2 in `out_dtype` from the gradients of
     the rotated tensors (expanded ones are summed over each GQA group first)."""
-    n = b_idx.shape[0]
     dq, dk, dv = dq.contiguous(), dk.contiguous(), dv.contiguous()
-    cos, sin = _tables(cos, sin)
-    dq_in = torch.empty(n, heads * HEAD_DIM, dtype=out_dtype, device=dq.device)
-    dk_in = torch.empty(n, kv_heads * HEAD_DIM, dtype=out_dtype, device=dq.device)
-    dv_in = torch.empty_like(dk_in)
-    scb, sct = _rope_strides(cos)
     if not (dq.dtype == dk.dtype == dv.dtype):
         raise ValueError("gradient dtypes differ")
-    check(lib().va_rope_bwd(_ptr(dq), _ptr(dk), _ptr(dv), _ptr(cos), _ptr(sin), scb, sct,
-                            _ptr(b_idx), _ptr(t_idx), _ptr(dq_in), _ptr(dk_in), _ptr(dv_in), n,
-                            heads, kv_heads, HEAD_DIM, seq, _DTYPES[dq.dtype], _DTYPES[out_dtype],
-                            layout, int(expand), _stream()), "va_rope_bwd")
+    return _rope_backward(_ptr(dq), _ptr(dk), _ptr(dv), dq.dtype, dq.device, cos, sin, b_idx,
+                          t_idx, heads, kv_heads, out_dtype, layout, expand, seq)
+
+
+def _rope_backward(dq, dk, dv, dtype, device, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype,
+                   layout, expand, seq):
+    """rope_backward of the gradients at the addresses dq, dk and dv, which the caller keeps."""
+    n = b_idx.shape[0]
+    cos, sin = _tables(cos, sin)
+    dq_in = torch.empty(n, heads * HEAD_DIM, dtype=out_dtype, device=device)
+    dk_in = torch.empty(n, kv_heads * HEAD_DIM, dtype=out_dtype, device=device)
+    dv_in = torch.empty_like(dk_in)
+    scb, sct = _rope_strides(cos)
+    check(lib().va_rope_bwd(dq, dk, dv, _ptr(cos), _ptr(sin), scb, sct, _ptr(b_idx), _ptr(t_idx),
+                            _ptr(dq_in), _ptr(dk_in), _ptr(dv_in), n, heads, kv_heads, HEAD_DIM,
+                            seq, _DTYPES[dtype], _DTYPES[out_dtype], layout, int(expand),
+                            _stream()), "va_rope_bwd")
     return dq_in, dk_in, dv_in
 
 
@@ -575,9 +611,8 @@ class PackedAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, cos, sin, b_idx, t_idx, seq, heads, kv_heads, lengths, scale,
                 offload):
-        with torch.no_grad():
-            out, lse, rot, plan = _attend(q, k, v, cos, sin, b_idx, t_idx, seq, heads, kv_heads,
-                                          lengths, scale)
+        out, lse, rot, plan = _attend(q, k, v, cos, sin, b_idx, t_idx, seq, heads, kv_heads,
+                                      lengths, scale)
         ctx.consts = (cos, sin, b_idx, t_idx)
         ctx.meta = (seq, heads, kv_heads, lengths, scale)
         ctx.dtypes = (q.dtype, k.dtype, v.dtype)
@@ -615,10 +650,12 @@ class PackedAttention(torch.autograd.Function):
         else:
             # dq and the per-query-head dK/dV partials; the inverse rotation sums the partials
             # over each GQA group in fp32 while it rotates (as attention.py:113-134 sums copies)
-            dq_r, dk_part, dv_part, _ws = attention_backward(dout, qr, kr, vr, out, lse, plan,
-                                                             scale, outputs=False)
-            dq, dk, dv = rope_backward(dq_r, dk_part, dv_part, cos, sin, b_idx, t_idx, heads,
-                                       kv_heads, q_dtype, expand=True)
+            dq_r, _, _, ws, offs = _attention_backward(dout, qr, kr, vr, out, lse, plan, scale,
+                                                       False)
+            part = _ptr(ws)
+            dq, dk, dv = _rope_backward(_ptr(dq_r), part + offs[0], part + offs[1], qr.dtype,
+                                        qr.device, cos, sin, b_idx, t_idx, heads, kv_heads,
+                                        q_dtype, _lib.VA_LAYOUT_PACKED, True, 0)
         grads = (dq.to(q_dtype), dk.to(k_dtype), dv.to(v_dtype))
         return (*grads, None, None, None, None, None, None, None, None, None, None)
 
