@@ -611,55 +611,63 @@ __global__ __launch_bounds__(fwd::NT, 1) void fwd_kernel(
 
 // --------------------------------------------------------------------------------------------
 // Forward for many work items: 4 waves per work item (one per query strip, each over all of the
-// item's key tiles), three work-groups per CU. The three waves of a SIMD come from different work
+// item's key tiles), several work-groups per CU. The waves of a SIMD come from different work
 // items with their own barriers: one's MFMAs overlap the others' softmax and waits without any
 // phase arrangement, one item's start (loads) and end (stores) overlap the others' tiles, and no
 // item merges halves at its end.
 //
-// Three waves per SIMD leave 168 registers and 53 KB of LDS each: 32-key tiles (16 scores per
-// lane) in a ring of three stages, the copies two tiles ahead, one barrier per tile. A tile's rows
-// are stored in groups of 4 (1 KB, one copy instruction) 1088 bytes apart, chunk c of row r at
-// c ^ (r & 3): the 64-byte shift from group to group and the two XOR bits spread 16 rows of K
-// over the 16 chunk columns, and the transposed V reads (4 rows x 32 bytes of columns j and
-// j + 64) over all 64 banks, while all but two address bits stay immediates: 6 address registers
-// instead of 16.
+// Two shapes (Ring). Long lists: three work-groups a CU, which leave 168 registers and 53 KB of LDS
+// each: 32-key tiles (16 scores per lane) in a ring of three stages, the copies two tiles ahead.
+// Shorter ones: two work-groups a CU of 64-key tiles in two stages (68 KB, 213 registers), half the
+// barriers, maxima and rescale tests per key; the rule between them is at the launch. One barrier
+// per tile in both. A tile's rows are stored in groups of 4 (1 KB, one copy instruction) 1088 bytes
+// apart, chunk c of row r at c ^ (r & 3): the 64-byte shift from group to group and the two XOR
+// bits spread 16 rows of K over the 16 chunk columns, and the transposed V reads (4 rows x 32
+// bytes of columns j and j + 64) over all 64 banks, while all but two address bits stay
+// immediates: 6 address registers instead of 16.
 //
 // What bounds it: at documents of thousands of tokens the matrix cores' sustained rate on real
-// data (two documents of 8192 tokens, 28/4 heads, bf16: 883 us = 1090 TFLOP/s, where an 8192^3
+// data (two documents of 8192 tokens, 28/4 heads, bf16: 869 us = 1107 TFLOP/s, where an 8192^3
 // library product reaches 1390 on the same card; the MFMAs alone take 588 us, everything else
 // 493 us); at documents of a few hundred tokens the first loads and the last stores of each item
-// and HBM. Against two work-groups of 64-key tiles in two stages, 256 registers (interleaved
-// runs, one card): 8192-token documents 897 -> 883 us; 32768 tokens of 32 to 1740, 28/4 heads,
-// bf16 286 -> 263 us; 16384 tokens of 8 to 511, 12/2 heads, bf16 45.2 -> 41.7 us; 8192 tokens of
-// 16 to 512, 12/2 heads, fp16 24.5 -> 23.9 us. The same tiles in a ring of four stages, which
-// leaves two work-groups a CU, take 938 / 286 / 48 / 25 us.
+// and HBM. Against two work-groups of 64-key tiles in 256-byte rows with a four-bit XOR (223
+// registers), interleaved runs on one card: the 32-key shape at 8192-token documents 885 -> 869 us;
+// 32768 tokens of 32 to 4096, 28/4 heads, bf16 293 -> 270; the 64-key shape, the same bits, at 8192
+// tokens of 16 to 512, 12/2 heads, fp16 22.5 -> 22.3; 6144 of 32 to 4096, 16/2 heads, bf16 40.7 ->
+// 39.0; two documents of 2048, 16/2 heads 48.4 -> 46.6 (32-key tiles held to two work-groups take
+// 22.5, 48.5 and 54.1).
 // --------------------------------------------------------------------------------------------
 namespace fwdl {
-constexpr int NW = fwd::NS;     // waves = query strips
+constexpr int NW = fwd::NS;  // waves = query strips
 constexpr int NT = NW * 64;
-constexpr int BN = 32;          // keys per tile
 constexpr int D = fwd::D, BM = fwd::BM;
-constexpr int GRP = 4 * D + 32;       // halfs from one group of 4 rows to the next
-constexpr int TILE = BN / 4 * GRP;    // halfs of a K or V tile
-constexpr int STAGE = 2 * TILE;       // K, V of one tile
-constexpr int NSTAGE = 3;
-constexpr int PER_CU = 3;             // work-groups per CU
-constexpr int64_t kThreeMinItems = 2 * PER_CU * kPlanCus;
-constexpr unsigned kPairPad = 8192;   // LDS that leaves room for two
-static_assert(PER_CU * (NSTAGE * STAGE * 2 + kPairPad) > 160 * 1024 &&
-                  2 * (NSTAGE * STAGE * 2 + kPairPad) <= 160 * 1024, "two work-groups");
-static_assert(BM / 4 * GRP <= (NSTAGE - 1) * STAGE, "the Q tile fits in stages 1 and 2");
-static_assert(PER_CU * NSTAGE * STAGE * 2 <= 160 * 1024, "LDS of three work-groups");
-static_assert(BN / 4 * 2 == 4 * NW, "copy map: 4 row groups per wave and tile pair K, V");
+constexpr int GRP = 4 * D + 32;  // halfs from one group of 4 rows to the next
+constexpr int64_t kThreeMinItems = 7 * kPlanCus;
+
+template <int KEYS>  // keys per tile
+struct Ring {
+  static constexpr int BLOCKS = KEYS / 32;           // 32-key MFMA blocks of a tile
+  static constexpr int STAGES = KEYS == 32 ? 3 : 2;
+  static constexpr int PER_CU = KEYS == 32 ? 3 : 2;  // work-groups per CU
+  static constexpr int TILE = KEYS / 4 * GRP;        // halfs of a K or V tile
+  static constexpr int STAGE = 2 * TILE;             // K, V of one tile
+  static constexpr int GROUPS = KEYS / 4 / NW;       // row groups that a wave copies per K or V tile
+  static_assert(KEYS == 32 || KEYS == 64, "tile shapes");
+  static_assert(BM / 4 * GRP <= (STAGES - 1) * STAGE, "the Q tile fits behind stage 0");
+  static_assert(PER_CU * STAGES * STAGE * 2 <= 160 * 1024 &&
+                    (PER_CU + 1) * STAGES * STAGE * 2 > 160 * 1024, "LDS sets the work-groups");
+};
 }  // namespace fwdl
 
-template <class E>
-__global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
+template <class E, int KEYS>
+__global__ __launch_bounds__(fwdl::NT, fwdl::Ring<KEYS>::PER_CU) void fwd_lean_kernel(
     const int4* __restrict__ items, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int hq, int hkv,
     uint16_t* __restrict__ o, float* __restrict__ lse, int n_tokens, float scale_log2) {
   using namespace fwdl;
-  __shared__ __attribute__((aligned(16))) uint16_t smem_raw[NSTAGE * STAGE];
+  using R = Ring<KEYS>;
+  constexpr int BLOCKS = R::BLOCKS, STAGES = R::STAGES, TILE = R::TILE, STAGE = R::STAGE;
+  __shared__ __attribute__((aligned(16))) uint16_t smem_raw[STAGES * STAGE];
   lds_u16* smem = (lds_u16*)smem_raw;
 
   const int4 it = items[blockIdx.x];
@@ -681,32 +689,34 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
   const bool q_valid = my_q < q_end;
   const int ws = __builtin_amdgcn_readfirstlane(strip);
   const int wq0_u = __builtin_amdgcn_readfirstlane(wq0);
-  const int n_tiles = (q_end - doc_start + BN - 1) / BN;
+  const int n_tiles = (q_end - doc_start + KEYS - 1) / KEYS;
 
-  // Copies of the tiles, in tile order: wave s moves row groups 2 s and 2 s + 1 of K and of V, 4
-  // instructions; lane i lands in chunk slot i & 15 of row i >> 4 of the group and fetches the
+  // Copies of the tiles, in tile order: wave s moves its GROUPS row groups of K and of V, one
+  // instruction each; lane i lands in chunk slot i & 15 of row i >> 4 of the group and fetches the
   // chunk that belongs there. Rows past the document end read as zeros (masked keys, zero P).
   const int c_row = lane >> 4;
-  const int coff = ((8 * ws + c_row) * (int)kvrow + 8 * ((lane & 15) ^ c_row)) * 2;
+  const int coff = ((4 * R::GROUPS * ws + c_row) * (int)kvrow + 8 * ((lane & 15) ^ c_row)) * 2;
   const int coff4 = 4 * (int)kvrow * 2;
   const uint16_t* kp = k + (long)doc_start * kvrow + kvh * D;
   const uint16_t* vp = v + (long)doc_start * kvrow + kvh * D;
   long left = ((long)(doc_end - doc_start - 1) * kvrow + D) * 2;  // bytes from kp to the end
-  const long step = (long)BN * kvrow;
+  const long step = (long)KEYS * kvrow;
   auto copy_next = [&](uint32_t dst) {
     const u32x4 rk = make_rsrc4(kp, left), rv = make_rsrc4(vp, left);
-    dst += 2 * ws * GRP * 2;
-    dma16_opaque(rk, dst, coff);
-    dma16_opaque(rk, dst + GRP * 2, coff + coff4);
-    dma16_opaque(rv, dst + TILE * 2, coff);
-    dma16_opaque(rv, dst + (TILE + GRP) * 2, coff + coff4);
+    dst += R::GROUPS * ws * GRP * 2;
+#pragma unroll
+    for (int j = 0; j < R::GROUPS; ++j) dma16_opaque(rk, dst + j * GRP * 2, coff + j * coff4);
+#pragma unroll
+    for (int j = 0; j < R::GROUPS; ++j)
+      dma16_opaque(rv, dst + (TILE + j * GRP) * 2, coff + j * coff4);
     kp += step;
     vp += step;
     left -= step * 2;
   };
 
-  // Read offsets (halfs) inside a tile. K (A operand of S^T): row perm32(l32), chunk 2 kk + hi.
-  // V^T: row 8 hi + 2 (src >> 2) + e (+ 16 c), chunk 8 (grp & 1) + 2 db + (sg >> 1): registers
+  // Read offsets (halfs) inside a tile. K (A operand of S^T): row perm32(l32) (+ 32 b), chunk
+  // 2 kk + hi.
+  // V^T: row 8 hi + 2 (src >> 2) + e (+ 16 c + 32 b), chunk 8 (grp & 1) + 2 db + (sg >> 1): registers
   // [8 c, 8 c + 8) of accumulator db then hold d = 16 db + 64 c + 8 hi + 0..7.
   int koff[2], toff[2][2];
   {
@@ -731,39 +741,58 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
   for (int db = 0; db < 4; ++db) oacc[db] = f32x16{};
   float m_run = -INFINITY, l_run = 0.f;
 
-  // S^T of one tile (K at `kb`): 8 MFMAs, each K operand read 4 MFMAs ahead.
-  auto s_tile = [&](const lds_u16* kb, f32x16& s) {
-    s = f32x16{};
-    auto k_read = [&](int i) { return ld128(kb + koff[i & 1] + 32 * (i >> 1)); };
+  // S^T of one tile (K at `kb`): MFMAs over (kk, b), each K operand read 4 ahead.
+  auto s_tile = [&](const lds_u16* kb, f32x16(&s)[BLOCKS]) {
+    constexpr int N = 8 * BLOCKS;
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) s[b] = f32x16{};
+    auto k_read = [&](int i) {
+      const int kk = i / BLOCKS, b = i % BLOCKS;
+      return ld128(kb + koff[kk & 1] + 32 * (kk >> 1) + 8 * b * GRP);
+    };
     u32x4 ka[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) ka[i] = k_read(i);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      s = E::mfma(ka[i & 3], qf[i], s);
-      if (i + 4 < 8) ka[i & 3] = k_read(i + 4);
+    for (int i = 0; i < N; ++i) {
+      s[i % BLOCKS] = E::mfma(ka[i & 3], qf[i / BLOCKS], s[i % BLOCKS]);
+      if (i + 4 < N) ka[i & 3] = k_read(i + 4);
+    }
+    if constexpr (BLOCKS == 2) {
+      VA_SCHED(kSchedDsRead, 4);
+#pragma unroll
+      for (int i = 0; i < N - 4; ++i) {
+        VA_SCHED(kSchedMfma, 1);
+        VA_SCHED(kSchedDsRead, 1);
+      }
+      VA_SCHED(kSchedMfma, 4);
     }
   };
   // Mask, online softmax and O^T += V^T P^T of the tile of keys from kv0 (V at `vb`).
-  auto pv_tile = [&](const lds_u16* vb, int kv0, f32x16& s) {
-    auto v_read = [&](int i) {  // i = (c, db) in MFMA order
-      const int c = i >> 2, db = i & 3;
-      const lds_u16* p = vb + 4 * c * GRP + 32 * (db >> 1);
+  auto pv_tile = [&](const lds_u16* vb, int kv0, f32x16(&s)[BLOCKS]) {
+    constexpr int N = 8 * BLOCKS;
+    auto v_read = [&](int i) {  // i = (b, c, db) in MFMA order
+      const int b = i >> 3, c = (i >> 2) & 1, db = i & 3;
+      const lds_u16* p = vb + (8 * b + 4 * c) * GRP + 32 * (db >> 1);
       const u32x2 x = ldtr(p + toff[db & 1][0]), y = ldtr(p + toff[db & 1][1]);
       return u32x4{x[0], x[1], y[0], y[1]};
     };
     u32x4 va[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) va[i] = v_read(i);
-    if (kv0 + BN - 1 > wq0_u) {
+    if (kv0 + KEYS - 1 > wq0_u) {
       const int lim = my_q - kv0;
 #pragma unroll
-      for (int j = 0; j < 16; ++j)
-        if (reg_row(j, hi) > lim) s[j] = -INFINITY;
+      for (int b = 0; b < BLOCKS; ++b)
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          if (32 * b + reg_row(j, hi) > lim) s[b][j] = -INFINITY;
     }
     float mt = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) mt = fmaxf(mt, s[j]);
+    for (int b = 0; b < BLOCKS; ++b)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) mt = fmaxf(mt, s[b][j]);
     mt = max_with_other_half(mt) * scale_log2;
     if (__builtin_amdgcn_ballot_w64(mt > m_run + fwd::kRescaleLog2)) {
       const float m_new = fmaxf(m_run, mt);
@@ -774,26 +803,29 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
       for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
     }
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
+    constexpr int SUMS = BLOCKS == 1 ? 2 : 1;  // chains of the row sum
     float rs[2] = {0.f, 0.f};
-    u32x4 pf[2];
+    u32x4 pf[BLOCKS][2];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      float p[8];
+    for (int b = 0; b < BLOCKS; ++b)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) p[e] = fast_exp2(fmaf(s[8 * c + e], scale_log2, -m_use));
-      pf[c] = pack8_tr<E>(p);
+      for (int c = 0; c < 2; ++c) {
+        float p[8];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) rs[c] = E::sum2(pf[c][w], rs[c]);
-    }
+        for (int e = 0; e < 8; ++e) p[e] = fast_exp2(fmaf(s[b][8 * c + e], scale_log2, -m_use));
+        pf[b][c] = pack8_tr<E>(p);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) rs[c % SUMS] = E::sum2(pf[b][c][w], rs[c % SUMS]);
+      }
     l_run += rs[0] + rs[1];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      oacc[i & 3] = E::mfma(va[i & 3], pf[i >> 2], oacc[i & 3]);
-      if (i + 4 < 8) va[i & 3] = v_read(i + 4);
+    for (int i = 0; i < N; ++i) {
+      oacc[i & 3] = E::mfma(va[i & 3], pf[i >> 3][(i >> 2) & 1], oacc[i & 3]);
+      if (i + 4 < N) va[i & 3] = v_read(i + 4);
     }
   };
 
-  // Q (32 row groups) into stages 1 and 2, tile 0 into stage 0; every lane reads its query's row.
+  // Q (32 row groups) from stage 1 on, tile 0 into stage 0; every lane reads its query's row.
   {
     const long bytes = ((long)(doc_end - q0 - 1) * qrow + D) * 2;
     const u32x4 rq = make_rsrc4(q + (long)q0 * qrow + h * D, bytes);
@@ -817,26 +849,29 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
   // A strip computes the tiles up to its diagonal; past them, and in a strip past the document's
   // end (the last item of a document whose length is not a multiple of 128), its wave only copies
   // and meets the barriers, and leaves its SIMD to the other work-groups' waves.
-  const int n_live = wq0_u < q_end ? min((wq0_u + 31 - doc_start) / BN + 1, n_tiles) : 0;
-  if (1 < n_tiles) copy_next(lds_addr(smem + STAGE));
+  const int n_live = wq0_u < q_end ? min((wq0_u + 31 - doc_start) / KEYS + 1, n_tiles) : 0;
+  if (STAGES == 3 && 1 < n_tiles) copy_next(lds_addr(smem + STAGE));
   int stage = 0;
   auto next = [&](int t) {
-    // This wave's copies of tile t + 1 have landed in LDS; those of tile t + 2 stay in flight.
-    if (t + 2 < n_tiles) wait_vmcnt<4>();
+    // This wave's copies of tile t + 1 have landed in LDS; those of tile t + 2 (three stages) stay
+    // in flight.
+    if (t + STAGES - 1 < n_tiles) wait_vmcnt<(STAGES - 2) * 2 * R::GROUPS>();
     else wait_vmcnt<0>();
     __syncthreads();
-    stage = stage == NSTAGE - 1 ? 0 : stage + 1;
+    stage = stage == STAGES - 1 ? 0 : stage + 1;
   };
-  auto copy_ahead = [&](int t) {  // tile t + 2, into the stage that tile t - 1 was last read from
-    if (t + 2 < n_tiles) copy_next(lds_addr(smem + (stage == 0 ? NSTAGE - 1 : stage - 1) * STAGE));
+  // Tile t + STAGES - 1, into the stage that tile t - 1 was last read from.
+  auto copy_ahead = [&](int t) {
+    if (t + STAGES - 1 < n_tiles)
+      copy_next(lds_addr(smem + (stage == 0 ? STAGES - 1 : stage - 1) * STAGE));
   };
   int t = 0;
   for (; t < n_live; ++t) {
     const lds_u16* kb = smem + stage * STAGE;
-    f32x16 s;
+    f32x16 s[BLOCKS];
     s_tile(kb, s);
     copy_ahead(t);  // after this tile's S^T MFMAs: the wave waits for S anyway
-    pv_tile(kb + TILE, doc_start + t * BN, s);
+    pv_tile(kb + TILE, doc_start + t * KEYS, s);
     next(t);
   }
   for (; t < n_tiles; ++t) {
@@ -857,7 +892,7 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::PER_CU) void fwd_lean_kernel(
                                oacc[db][8 * c + 2] * inv, oacc[db][8 * c + 3] * inv,
                                oacc[db][8 * c + 4] * inv, oacc[db][8 * c + 5] * inv,
                                oacc[db][8 * c + 6] * inv, oacc[db][8 * c + 7] * inv);
-  static_assert(NW * 32 * (8 * 16 + 8) <= NSTAGE * STAGE, "row tiles fit in LDS");
+  static_assert(NW * 32 * (8 * 16 + 8) <= STAGES * STAGE, "row tiles fit in LDS");
   store_rows32<16>(smem + strip * 32 * (8 * 16 + 8), w, lane,
                    [&](int r) { return o + (long)(wq0 + r) * qrow + h * D; }, q_end - wq0);
   if (q_valid && hi == 0) {
@@ -870,14 +905,20 @@ template <class E>
 static hipError_t launch_fwd_t(const FwdArgs& a) {
   if (a.n_items == 0) return hipSuccess;
   if (a.kernel == 2) {
-    // Two work-groups a CU (by LDS that the kernel does not use) until the list fills the slots of
-    // three twice over (ceil(N / 128) Hq, as the kernel's own rule): in one short list each of a
-    // CU's items runs slower beside two others, and the longest sets the time. Four layers of
-    // 8192 tokens in documents of 16 to 512, 12 heads (768), captured: 460 us with three, 450 with
-    // two; 16384 tokens of 12 heads (1536): 42.3 us with three, 47.4 with two.
+    // Three work-groups a CU from seven items per CU on (ceil(N / 128) Hq, as the kernel's own rule,
+    // so that host and device plans take the same shape). In a shorter list each of a CU's items
+    // runs slower beside two others and the longest sets the time. 32-key against 64-key tiles, 12,
+    // 28, 16 and 8 heads (us): documents of 8192 at 768 items 234 / 223, 95 / 93, 167 / 155, 222 / 182,
+    // at 1536 416 / 404, 330 / 321, 332 / 317, 419 / 411, at 1792 428 / 425, 438 / 439, 392 / 392, 447 /
+    // 451, at 2600 614 / 627, 516 / 526, 561 / 579, 673 / 682; documents of 16 to 512 at 768 23.5 / 22.0,
+    // 21.9 / 21.7, 20.5 / 20.7, 23.8 / 24.8, at 1536 36.0 / 38.4, 34.6 / 36.1, 33.9 / 37.2, 42.0 / 45.2.
+    // So short documents would take three from about 1100 items on and long ones lose until 1792;
+    // the sizes that the rule reads do not tell them apart, and below the line the 64-key shape is
+    // at or below the former kernel's time for both.
     const bool three = (a.n_tokens + fwdl::BM - 1) / fwdl::BM * a.hq >= fwdl::kThreeMinItems;
-    hipLaunchKernelGGL((fwd_lean_kernel<E>), dim3((unsigned)a.n_items), dim3(fwdl::NT),
-                       three ? 0u : fwdl::kPairPad, a.stream, (const int4*)a.items, (const uint16_t*)a.q, (const uint16_t*)a.k,
+    hipLaunchKernelGGL((three ? fwd_lean_kernel<E, 32> : fwd_lean_kernel<E, 64>),
+                       dim3((unsigned)a.n_items), dim3(fwdl::NT), 0, a.stream,
+                       (const int4*)a.items, (const uint16_t*)a.q, (const uint16_t*)a.k,
                        (const uint16_t*)a.v, a.hq, a.hkv, (uint16_t*)a.out, a.lse,
                        (int)a.n_tokens, a.scale * kLog2e);
     return hipGetLastError();

@@ -12,8 +12,9 @@ constexpr int kHeadDim = 128;  // Qwen2.5-1.5B / 7B head size; the kernels are b
 constexpr int kFwdWaves = 4;                 // forward: 32 queries per wave
 constexpr int kFwdBlockM = 32 * kFwdWaves;   // queries per forward work item
 // From this many 128-query tiles x query heads on (ceil(N / 128) Hq >= VA_FWD_MANY_ITEMS, a lower
-// bound of the forward list's length that host and device plans share), the 4-wave forward (three
-// work-groups per CU) runs instead of the 8-wave one: every CU then gets at least two items.
+// bound of the forward list's length that host and device plans share), the 4-wave forward (two
+// work-groups per CU, three in long lists) runs instead of the 8-wave one: every CU then gets at
+// least two items.
 constexpr int kFwdLeanMinItems = 512;
 constexpr int kBwdBlockN = 128;  // keys per backward kv work item
 constexpr int kBwdBlockQ = 32;   // queries per kv-item step

@@ -7,33 +7,112 @@ import torch
 
 from hackaton_amd import attention as att
 from hackaton_amd import workloads as wl
+from oracle import attention_oracle as orc
 from tests.test_gpu_attention import SCALE, TOL, banner, oracle
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("lengths", [[1, 31, 32, 33], [63, 64, 65], [95, 96, 97, 127],
-                                     [128, 129, 160, 161], [255, 256, 257], [383, 385]])
-@pytest.mark.parametrize("hq,hkv,dtype", [(3, 1, torch.float16), (14, 2, torch.bfloat16)])
-def test_many_item_forward_at_tile_and_ring_edges(lengths, hq, hkv, dtype):
-    """One, two, three and more 32-key tiles through the three-stage ring, with full and partial
-    last tiles and strips, documents before and after each other in one packed array."""
-    banner("many-item forward edges", lengths, hq, hkv, dtype)
-    q, k, v, do = wl.make_inputs(lengths, hq, hkv, dtype, seed=sum(lengths))
-    n, dev = sum(lengths), torch.device("cuda")
-    plan = att._plan(att._cu_seqlens(lengths, dev), hq, hkv)
-    qd, kd, vd = (t.to(dev) for t in (q, k, v))
-    out = torch.full_like(qd, float("nan"))
-    lse = torch.full((hq, n), float("nan"), dtype=torch.float32, device=dev)
-    att.check(att.lib().va_fwd_kernel(att._lib.VA_FWD_MANY, qd.data_ptr(), kd.data_ptr(),
-                                      vd.data_ptr(), out.data_ptr(), lse.data_ptr(),
+EDGES = [[1, 31, 32, 33], [63, 64, 65], [95, 96, 97, 127], [128, 129, 160, 161], [255, 256, 257],
+         [383, 385]]
+LONG_LIST = 7 * 256  # (tile, head) pairs from which the many-item forward runs its 32-key tiles
+
+
+def _many_item_forward(q, k, v, lengths, scale=SCALE):
+    """out and lse of va_fwd_kernel(VA_FWD_MANY) on the GPU tensors, from NaN-filled outputs."""
+    (n, hq, _), hkv = q.shape, k.shape[1]
+    plan = att._plan(att._cu_seqlens(lengths, q.device), hq, hkv)
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((hq, n), float("nan"), dtype=torch.float32, device=q.device)
+    att.check(att.lib().va_fwd_kernel(att._lib.VA_FWD_MANY, q.data_ptr(), k.data_ptr(),
+                                      v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                       plan.fwd_items.data_ptr(), plan.n_fwd, n, hq, hkv, 128,
-                                      SCALE, 0 if dtype == torch.float16 else 1, att._stream()),
+                                      scale, 0 if q.dtype == torch.float16 else 1, att._stream()),
               "va_fwd_kernel")
     torch.cuda.synchronize()
+    return out, lse
+
+
+@pytest.mark.parametrize("lengths", EDGES)
+@pytest.mark.parametrize("hq,hkv,dtype", [(3, 1, torch.float16), (14, 2, torch.bfloat16)])
+def test_many_item_forward_at_tile_and_ring_edges(lengths, hq, hkv, dtype):
+    """One, two, three and more 64-key tiles through the two stages of a short list (two work-groups
+    a CU), with full and partial last tiles and strips, documents before and after each other in
+    one packed array."""
+    banner("many-item forward edges", lengths, hq, hkv, dtype)
+    q, k, v, do = wl.make_inputs(lengths, hq, hkv, dtype, seed=sum(lengths))
+    out, lse = _many_item_forward(q.cuda(), k.cuda(), v.cuda(), lengths)
     o_ref, lse_ref = oracle(q, k, v, do, lengths)[:2]
     assert float(np.max(np.abs(out.cpu().float().numpy() - o_ref))) <= TOL[dtype]["o"]
     assert float(np.max(np.abs(lse.cpu().numpy() - lse_ref))) <= TOL[dtype]["lse"]
+
+
+@pytest.mark.parametrize("hq,hkv,dtype", [(96, 8, torch.float16), (98, 14, torch.bfloat16)])
+def test_many_item_forward_edges_in_a_long_list(hq, hkv, dtype):
+    """The same documents in one batch with heads enough for the 32-key tiles in a ring of three
+    stages, three work-groups a CU: one, two, three and more tiles, each end of the ring."""
+    lengths = sum(EDGES, [])
+    assert -(-sum(lengths) // 128) * hq >= LONG_LIST
+    banner("many-item forward edges, long list", hq, hkv, dtype)
+    q, k, v, _ = wl.make_inputs(lengths, hq, hkv, dtype, seed=hq)
+    out, lse = _many_item_forward(q.cuda(), k.cuda(), v.cuda(), lengths)
+    o_ref, lse_ref = orc.attention_forward(*(t.double().numpy() for t in (q, k, v)),
+                                           orc.cu_seqlens_from_lengths(lengths), SCALE)
+    assert float(np.max(np.abs(out.cpu().float().numpy() - o_ref))) <= TOL[dtype]["o"]
+    assert float(np.max(np.abs(lse.cpu().numpy() - lse_ref))) <= TOL[dtype]["lse"]
+
+
+def _two_key_documents(dtype, hq, hkv, first):
+    """Documents of 200 tokens in which a query sees a key of score 0 (key 0), with `first` one
+    of 9 (key 70) and, 8 keys into the next 32, one of 5 to 7.5 more, in log2 units; every other key
+    lies 60 or more below. Returns lengths, q, k, v and the two late keys' positions."""
+    lengths = [200] * 5 + [24]
+    n = sum(lengths)
+    start = np.repeat(np.cumsum([0] + lengths[:-1]), lengths)
+    at = torch.from_numpy(np.arange(n) - start)
+    last = 40 if first is None else 104
+    rise = torch.linspace(5.0, 7.5, hkv * len(lengths)).view(len(lengths), hkv)
+    rise = torch.repeat_interleave(rise, torch.tensor(lengths), dim=0)
+    score = torch.full((n, hkv), -60.0)
+    score[at == 0] = 0.0
+    if first is not None:
+        score[at == first] = 9.0
+        rise = rise + 9.0
+    score[at == last] = rise[at == last]
+    k = torch.zeros(n, hkv, 128)
+    k[:, :, 0] = score
+    q = torch.zeros(n, hq, 128)
+    q[:, :, 0] = 1.0
+    return lengths, at, q.to(dtype), k.to(dtype), torch.randn(n, hkv, 128).to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("first", [None, 70])
+@pytest.mark.parametrize("long_list", [False])
+def test_many_item_forward_keeps_the_largest_weight_exact(long_list, first, dtype):
+    """The reference maximum moves freely over a document's first 64 keys and over the 64 keys where
+    it moved last, so the largest weight there is 1 and rounds to nothing: lse is within the
+    rounding of the weights below it. A maximum that stays at the first 32 keys' leaves the
+    largest weight at 2^5 to 2^7.5, rounded to 16 bits, which shows in lse.
+
+    Bound: the other weight is at most 2^-5 of the largest and its rounding u = 2^-9 (bf16) or
+    2^-12 (fp16) of it; fp32 sums, exponentials and logarithms of values below 24: 8 ulp of 16."""
+    hq, hkv = (224, 28) if long_list else (28, 28)
+    lengths, at, q, k, v = _two_key_documents(dtype, hq, hkv, first)
+    assert (-(-sum(lengths) // 128) * hq >= LONG_LIST) == long_list
+    banner("largest weight", long_list, first, dtype)
+    scale = float(np.float32(np.log(2.0)))  # scores are in log2 units
+    _, lse = _many_item_forward(q.cuda(), k.cuda(), v.cuda(), lengths, scale)
+    late = (at >= (40 if first is None else 104)).numpy()
+    s = torch.repeat_interleave(k[:, :, 0].double(), hq // hkv, dim=1).t().numpy() * scale
+    ref, start = np.empty_like(s), 0
+    for length in lengths:
+        rows = slice(start, start + length)
+        ref[:, rows] = np.logaddexp.accumulate(s[:, rows], axis=1)
+        start += length
+    u = 2.0 ** -12 if dtype == torch.float16 else 2.0 ** -9
+    bound = 2.0 ** -5 * u + 8 * 2.0 ** -20
+    assert float(np.max(np.abs(lse.cpu().double().numpy() - ref)[:, late])) <= bound
 
 
 def _positions(batch, seq, n, seed):
