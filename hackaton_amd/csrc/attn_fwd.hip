@@ -627,12 +627,12 @@ __global__ __launch_bounds__(fwd::NT, 1) void fwd_kernel(
 // immediates: 6 address registers instead of 16.
 //
 // What bounds it: at documents of thousands of tokens the matrix cores' sustained rate on real
-// data (two documents of 8192 tokens, 28/4 heads, bf16: 869 us = 1107 TFLOP/s, where an 8192^3
+// data (two documents of 8192 tokens, 28/4 heads, bf16: 875 us = 1099 TFLOP/s, where an 8192^3
 // library product reaches 1390 on the same card; the MFMAs alone take 588 us, everything else
 // 493 us); at documents of a few hundred tokens the first loads and the last stores of each item
 // and HBM. Against two work-groups of 64-key tiles in 256-byte rows with a four-bit XOR (223
-// registers), interleaved runs on one card: the 32-key shape at 8192-token documents 885 -> 869 us;
-// 32768 tokens of 32 to 4096, 28/4 heads, bf16 293 -> 270; the 64-key shape, the same bits, at 8192
+// registers), interleaved runs on one card: the 32-key shape at 8192-token documents 885 -> 875 us;
+// 32768 tokens of 32 to 4096, 28/4 heads, bf16 293 -> 274; the 64-key shape, the same bits, at 8192
 // tokens of 16 to 512, 12/2 heads, fp16 22.5 -> 22.3; 6144 of 32 to 4096, 16/2 heads, bf16 40.7 ->
 // 39.0; two documents of 2048, 16/2 heads 48.4 -> 46.6 (32-key tiles held to two work-groups take
 // 22.5, 48.5 and 54.1).
@@ -740,6 +740,8 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::Ring<KEYS>::PER_CU) void fwd_lean_k
 #pragma unroll
   for (int db = 0; db < 4; ++db) oacc[db] = f32x16{};
   float m_run = -INFINITY, l_run = 0.f;
+  constexpr float kMargin = KEYS == 32 ? 6.f : fwd::kRescaleLog2;
+  float margin = kMargin;
 
   // S^T of one tile (K at `kb`): MFMAs over (kk, b), each K operand read 4 ahead.
   auto s_tile = [&](const lds_u16* kb, f32x16(&s)[BLOCKS]) {
@@ -794,7 +796,19 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::Ring<KEYS>::PER_CU) void fwd_lean_k
 #pragma unroll
       for (int j = 0; j < 16; ++j) mt = fmaxf(mt, s[b][j]);
     mt = max_with_other_half(mt) * scale_log2;
-    if (__builtin_amdgcn_ballot_w64(mt > m_run + fwd::kRescaleLog2)) {
+    // The reference maximum moves (to every lane's exact one) when some lane's tile maximum exceeds
+    // it by more than 2^margin. A weight of 1 is exact in 16 bits, one near 2^margin is rounded, so
+    // the keys that set the maximum decide the error: with the 64-key tiles' 2^8, 32-key ones lose
+    // up to 1.5% in O and 3 to 20% in lse. With 2^6, and freely on the tile after a move, so that
+    // the start of a document and every move cover 64 keys again, O and lse are closer to 64 bits
+    // than the 64-key tiles' over 21 batches (documents of 33 to 8192, q and k times 1 to 5): 32768
+    // tokens, 28/4 heads, bf16, O 1.973e-3 with 64 keys, 1.990e-3 without this, 1.965e-3 with it,
+    // lse 1.91e-4, 1.97e-4, 1.89e-4; 16384 tokens, 12/2 heads, times 3, lse 3.92e-4, 4.73e-4, 3.35e-4.
+    // The rescales cost 1% (28/4 heads, 32768 tokens 270 -> 274 us; two documents of 8192 869 -> 875),
+    // 2 to 3% at 2048 keys and more with q and k times 2 to 5 (16/2 heads, 283 -> 289).
+    const bool moves = __builtin_amdgcn_ballot_w64(mt > m_run + margin) != 0;
+    if (KEYS == 32) margin = moves && margin > 0.f ? 0.f : kMargin;
+    if (moves) {
       const float m_new = fmaxf(m_run, mt);
       const float alpha = fast_exp2(m_run - (m_new == -INFINITY ? 0.f : m_new));
       m_run = m_new;
@@ -908,10 +922,10 @@ static hipError_t launch_fwd_t(const FwdArgs& a) {
     // Three work-groups a CU from seven items per CU on (ceil(N / 128) Hq, as the kernel's own rule,
     // so that host and device plans take the same shape). In a shorter list each of a CU's items
     // runs slower beside two others and the longest sets the time. 32-key against 64-key tiles, 12,
-    // 28, 16 and 8 heads (us): documents of 8192 at 768 items 234 / 223, 95 / 93, 167 / 155, 222 / 182,
-    // at 1536 416 / 404, 330 / 321, 332 / 317, 419 / 411, at 1792 428 / 425, 438 / 439, 392 / 392, 447 /
-    // 451, at 2600 614 / 627, 516 / 526, 561 / 579, 673 / 682; documents of 16 to 512 at 768 23.5 / 22.0,
-    // 21.9 / 21.7, 20.5 / 20.7, 23.8 / 24.8, at 1536 36.0 / 38.4, 34.6 / 36.1, 33.9 / 37.2, 42.0 / 45.2.
+    // 28, 16 and 8 heads (us): documents of 8192 at 768 items 236 / 223, 96 / 93, 168 / 155, 222 / 182,
+    // at 1536 418 / 404, 332 / 321, 333 / 317, 422 / 411, at 1792 431 / 425, 441 / 439, 395 / 392, 450 /
+    // 451, at 2600 617 / 627, 521 / 526, 568 / 579, 681 / 682; documents of 16 to 512 at 768 23.3 / 22.0,
+    // 22.8 / 21.7, 20.7 / 20.7, 23.7 / 24.8, at 1536 36.6 / 38.4, 34.7 / 36.1, 34.3 / 37.2, 42.2 / 45.2.
     // So short documents would take three from about 1100 items on and long ones lose until 1792;
     // the sizes that the rule reads do not tell them apart, and below the line the 64-key shape is
     // at or below the former kernel's time for both.

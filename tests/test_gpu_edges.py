@@ -88,7 +88,7 @@ def _two_key_documents(dtype, hq, hkv, first):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("first", [None, 70])
-@pytest.mark.parametrize("long_list", [False])
+@pytest.mark.parametrize("long_list", [False, True])
 def test_many_item_forward_keeps_the_largest_weight_exact(long_list, first, dtype):
     """The reference maximum moves freely over a document's first 64 keys and over the 64 keys where
     it moved last, so the largest weight there is 1 and rounds to nothing: lse is within the
