@@ -66,7 +66,6 @@ def _attn_dtype(t):
 # cu_seqlens and work plans
 # ------------------------------------------------------------------------------------------------
 _CU_SEQLENS = {}
-_PLANS = {}
 
 
 def _cu_seqlens(lengths, device):
@@ -83,7 +82,7 @@ def _cu_seqlens(lengths, device):
             offsets.append(offsets[-1] + int(length))
         cu = torch.tensor(offsets, dtype=torch.int32, device=device)
         cu._va_offsets = tuple(offsets)
-        cu._va_host_plans = {}  # (Hq, Hkv) -> Plan, beside the offsets that they are made from
+        cu._va_host_plans = {}  # (Hq, Hkv) -> Plan: found without a second hash of the offsets
         _CU_SEQLENS[key] = cu
     return cu
 
@@ -239,25 +238,27 @@ def _device_plan(lengths, n_tokens, hq, hkv):
     return plan
 
 
+# The plans of the last 33 (document offsets, heads) outlive the cu_seqlens tensors, of which fewer
+# are kept: a program that cycles through that many batches plans and uploads each one once.
+@functools.lru_cache(maxsize=33)
+def _host_plan(offsets, hq, hkv, device):
+    return Plan(offsets, hq, hkv, device)
+
+
 def _plan(cu_seqlens, hq, hkv):
     known = getattr(cu_seqlens, "_va_host_plans", None)
     if known is not None:
         plan = known.get((hq, hkv))
         if plan is None:
-            plan = known[(hq, hkv)] = Plan(cu_seqlens._va_offsets, hq, hkv, cu_seqlens.device)
+            plan = known[(hq, hkv)] = _host_plan(cu_seqlens._va_offsets, hq, hkv,
+                                                 cu_seqlens.device)
         return plan
     device_plan = getattr(cu_seqlens, "_va_plan", None)
     if device_plan is not None:
         return device_plan
     # a cu_seqlens tensor not made by _cu_seqlens: read it (one sync)
     offsets = tuple(int(x) for x in cu_seqlens.cpu().tolist())
-    key = (cu_seqlens.device, offsets, hq, hkv)
-    plan = _PLANS.get(key)
-    if plan is None:
-        if len(_PLANS) > 32:
-            _PLANS.clear()
-        plan = _PLANS[key] = Plan(offsets, hq, hkv, cu_seqlens.device)
-    return plan
+    return _host_plan(offsets, hq, hkv, cu_seqlens.device)
 
 
 # ------------------------------------------------------------------------------------------------
