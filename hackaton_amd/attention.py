@@ -245,6 +245,28 @@ def _host_plan(offsets, hq, hkv, device):
     return Plan(offsets, hq, hkv, device)
 
 
+# Host plans that a captured graph reads: its kernels hold the addresses of the work lists, and nothing
+# that lives as long as the graph holds the lists, so they stay until release_captured_plans(): 16
+# bytes per work item (50 KB for 8192 tokens of 12 heads), once for all layers of a graph.
+_CAPTURED_PLANS = set()
+
+
+def _capturing():
+    return torch.cuda.is_initialized() and torch._C._cuda_isCurrentStreamCapturing()
+
+
+def release_captured_plans():
+    """Give back the work lists kept for captured graphs. Only for a program that will replay none of
+    the graphs that it has captured with host lengths so far."""
+    _CAPTURED_PLANS.clear()
+
+
+def _kept(plan):
+    if plan not in _CAPTURED_PLANS and _capturing():
+        _CAPTURED_PLANS.add(plan)
+    return plan
+
+
 def _plan(cu_seqlens, hq, hkv):
     known = getattr(cu_seqlens, "_va_host_plans", None)
     if known is not None:
@@ -252,13 +274,13 @@ def _plan(cu_seqlens, hq, hkv):
         if plan is None:
             plan = known[(hq, hkv)] = _host_plan(cu_seqlens._va_offsets, hq, hkv,
                                                  cu_seqlens.device)
-        return plan
+        return _kept(plan)
     device_plan = getattr(cu_seqlens, "_va_plan", None)
     if device_plan is not None:
         return device_plan
     # a cu_seqlens tensor not made by _cu_seqlens: read it (one sync)
     offsets = tuple(int(x) for x in cu_seqlens.cpu().tolist())
-    return _host_plan(offsets, hq, hkv, cu_seqlens.device)
+    return _kept(_host_plan(offsets, hq, hkv, cu_seqlens.device))
 
 
 # ------------------------------------------------------------------------------------------------

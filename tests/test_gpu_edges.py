@@ -115,6 +115,49 @@ def test_many_item_forward_keeps_the_largest_weight_exact(long_list, first, dtyp
     assert float(np.max(np.abs(lse.cpu().double().numpy() - ref)[:, late])) <= bound
 
 
+def test_graph_with_host_lengths_outlives_the_plan_caches():
+    """A training step captured with host lengths, its autograd nodes gone, replays its own work lists
+    after 40 other batches have gone through the plan caches and the allocator."""
+    banner("captured plan")
+    lengths, hq, hkv = [200, 77, 31], 12, 2
+    dev = torch.device("cuda")
+    q, k, v, do = (t.to(dev) for t in wl.make_inputs(lengths, hq, hkv, torch.float16, seed=3))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    do = do.reshape(sum(lengths), -1)
+
+    def step():
+        out = att.varlen_attention(*leaves, lengths, SCALE)
+        return (out.detach(), *torch.autograd.grad(out, leaves, do))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        eager = [t.clone() for t in step()]
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    plan = att._plan(att._cu_seqlens(lengths, dev), hq, hkv)
+    addresses = {plan.fwd_items.data_ptr(), plan.bwd_items.data_ptr()}
+    del plan
+    others = []
+    for i in range(40):
+        cu = att._cu_seqlens([150 + i, 60], dev)
+        other = att._plan(cu, hq, hkv)
+        others += [other.fwd_items, other.bwd_items, torch.full_like(other.fwd_items, -1)]
+    assert not addresses & {t.data_ptr() for t in others}
+    for _ in range(2):
+        for t in captured:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(captured, eager):
+            assert torch.equal(x, y)
+    del graph, captured
+    att.release_captured_plans()
+
+
 def _positions(batch, seq, n, seed):
     """n distinct rows of a (batch, seq) batch in random order: (b_idx, t_idx) int32, on the GPU."""
     rows = torch.from_numpy(np.random.default_rng(seed).permutation(batch * seq)[:n])
