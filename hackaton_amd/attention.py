@@ -491,7 +491,7 @@ def rope_forward(q, k, v, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype, la
         raise ValueError(f"q, k and v must share a dtype, got {q.dtype}, {k.dtype}, {v.dtype}")
     v_as_is = layout == _lib.VA_LAYOUT_PACKED and not expand and v.dtype == out_dtype
     scb, sct = _rope_strides(cos)
-    if layout == _lib.VA_LAYOUT_PADDED:  # every row written by the kernel, zeros included
+    if layout == _lib.VA_LAYOUT_PADDED and expand:  # the kernel writes every row, zeros included
         qo = torch.empty(batch, heads, seq, HEAD_DIM, dtype=out_dtype, device=q.device)
         ko, vo = torch.empty_like(qo), torch.empty_like(qo)
         row_map = torch.empty(batch * seq, dtype=torch.int32, device=q.device)
@@ -500,6 +500,7 @@ def rope_forward(q, k, v, cos, sin, b_idx, t_idx, heads, kv_heads, out_dtype, la
             _ptr(row_map), _ptr(qo), _ptr(ko), _ptr(vo), n, batch, heads, kv_heads, HEAD_DIM, seq,
             _DTYPES[q.dtype], _DTYPES[out_dtype], _stream()), "va_rope_fwd_padded")
         return qo, ko, vo
+    # (the padded layout without expansion goes on to va_rope_fwd, which refuses it)
     qo = torch.empty(n, heads, HEAD_DIM, dtype=out_dtype, device=q.device)
     ko = torch.empty(n, kvo, HEAD_DIM, dtype=out_dtype, device=q.device)
     vo = v.view(n, kv_heads, HEAD_DIM) if v_as_is else torch.empty_like(ko)

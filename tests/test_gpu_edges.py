@@ -212,3 +212,17 @@ def test_padded_rotation_matches_the_packed_one(batch, seq, n, heads, kv_heads, 
         ref = torch.zeros(batch, heads, seq, 128, dtype=torch.float16, device="cuda")
         ref[b.long(), :, t.long()] = rows
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(4, 2), (2, 2)])
+def test_padded_rotation_without_expansion_is_refused(heads, kv_heads):
+    """rope_forward into the padded layout repeats key/value heads or raises; it does not expand what
+    it was told not to."""
+    b, t = _positions(2, 5, 3, seed=0)
+    q = torch.randn(3, heads * 128, device="cuda").half()
+    k, v = (torch.randn(3, kv_heads * 128, device="cuda").half() for _ in range(2))
+    cos = torch.ones(1, 5, 128, device="cuda")
+    with pytest.raises(att._lib.VarlenAttnError) as e:
+        att.rope_forward(q, k, v, cos, cos, b, t, heads, kv_heads, torch.float16,
+                         att._lib.VA_LAYOUT_PADDED, False, 2, 5)
+    assert e.value.code == att._lib.VA_EINVAL
