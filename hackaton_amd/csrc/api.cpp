@@ -224,7 +224,7 @@ namespace {
 
 // Sizes of a padded tensor whose every row is written (row_map of batch * seq entries).
 int check_padded(int32_t batch, int32_t seq, int32_t heads, const char* what) {
-  if (batch < 0 || seq <= 0 || heads <= 0 || (int64_t)batch * seq > INT32_MAX)
+  if (batch < 0 || seq <= 0 || heads <= 0 || (int64_t)batch * seq > va::kMaxPaddedRows)
     return va::fail(VA_ESHAPE, "%s: batch=%d seq=%d heads=%d out of range", what, batch, seq, heads);
   return VA_OK;
 }

@@ -221,6 +221,12 @@ __device__ inline int token_at(const int32_t* row_map, const int32_t* b_idx, con
   return b_idx[pid] == b && t_idx[pid] == t ? pid : -1;
 }
 
+// This wave's row of a row_grid launch.
+__device__ inline long grid_row(int per_group) {
+  return ((long)blockIdx.y * gridDim.x + blockIdx.x) * per_group +
+         __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+
 // Each lane group handles two rows per pass: both rows, then the token's cos / sin chunks, are
 // loaded before either row is stored, so a wave has the reads of 16 rows in flight (all 16 rows
 // of a 12 + 2 + 2 head token in one pass). The tables are read again per pass, from cache.
@@ -253,8 +259,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_fwd_kernel(RopeArgs a) {
 // 107 MB tensors) and the rotation took 92 us, the row map and this kernel 81 us (396 MB, 4.9 TB/s).
 template <int IN, int OUT>
 __global__ __launch_bounds__(kRopeThreads) void rope_fwd_padded_kernel(RopeArgs a) {
-  const long row =
-      (long)blockIdx.x * kTokensPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long row = grid_row(kTokensPerGroup);
   if (row >= (long)a.batch * a.seq) return;
   const int b = (int)(row / a.seq), t = (int)(row - (long)b * a.seq);
   const int pid = token_at(a.row_map, a.b_idx, a.t_idx, (int)a.n_tokens, row, b, t);
@@ -375,8 +380,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_rows_kernel(
     const u32x4* __restrict__ src, u32x4* __restrict__ dst, const int32_t* __restrict__ b_idx,
     const int32_t* __restrict__ t_idx, long n_tokens, int heads, int seq, int row_chunks,
     int mode) {
-  const long pid =
-      (long)blockIdx.x * kPackWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long pid = grid_row(kPackWaves);
   if (pid >= n_tokens) return;
   const int total = heads * row_chunks;
   const long padded0 = (long)b_idx[pid] * heads * seq + t_idx[pid];
@@ -404,8 +408,7 @@ __global__ __launch_bounds__(kPackThreads) void unpack_rows_kernel(
     const u32x4* __restrict__ src, u32x4* __restrict__ dst, const int32_t* __restrict__ row_map,
     const int32_t* __restrict__ b_idx, const int32_t* __restrict__ t_idx, int n_tokens, long rows,
     int heads, int seq, int row_chunks) {
-  const long row =
-      (long)blockIdx.x * kPackWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long row = grid_row(kPackWaves);
   if (row >= rows) return;
   const int b = (int)(row / seq), t = (int)(row - (long)b * seq);
   const int pid = token_at(row_map, b_idx, t_idx, n_tokens, row, b, t);
@@ -432,10 +435,9 @@ template <int IN, int OUT>
 hipError_t launch_rope_t(const RopeArgs& a, bool fwd) {
   const unsigned groups = (unsigned)((a.n_tokens + kTokensPerGroup - 1) / kTokensPerGroup);
   if (fwd && a.row_map != nullptr) {
-    const long rows = (long)a.batch * a.seq;
     hipLaunchKernelGGL((rope_fwd_padded_kernel<IN, OUT>),
-                       dim3((unsigned)((rows + kTokensPerGroup - 1) / kTokensPerGroup)),
-                       dim3(kRopeThreads), 0, a.stream, a);
+                       row_grid((int64_t)a.batch * a.seq, kTokensPerGroup), dim3(kRopeThreads), 0,
+                       a.stream, a);
   } else if (fwd) {
     hipLaunchKernelGGL((rope_fwd_kernel<IN, OUT>), dim3(groups), dim3(kRopeThreads), 0, a.stream,
                        a);
@@ -474,7 +476,7 @@ hipError_t launch_pack_rows(const void* src, void* dst, const int32_t* b_idx, co
                             hipStream_t stream) {
   if (n_tokens == 0) return hipSuccess;
   const int chunks = row_bytes / 16;
-  const dim3 grid((unsigned)((n_tokens + kPackWaves - 1) / kPackWaves));
+  const dim3 grid = row_grid(n_tokens, kPackWaves);
   const auto kernel = chunks == 16   ? pack_rows_kernel<4>
                       : chunks == 32 ? pack_rows_kernel<5>
                                      : pack_rows_kernel<-1>;
@@ -497,7 +499,7 @@ hipError_t launch_unpack_rows(const void* src, void* dst, const int32_t* row_map
   const long rows = (long)batch * seq;
   if (rows == 0) return hipSuccess;
   const int chunks = row_bytes / 16;
-  const dim3 grid((unsigned)((rows + kPackWaves - 1) / kPackWaves));
+  const dim3 grid = row_grid(rows, kPackWaves);
   const auto kernel = chunks == 16   ? unpack_rows_kernel<4>
                       : chunks == 32 ? unpack_rows_kernel<5>
                                      : unpack_rows_kernel<-1>;

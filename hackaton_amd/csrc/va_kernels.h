@@ -156,6 +156,18 @@ hipError_t launch_rope_bwd(const RopeArgs& a);
 hipError_t launch_pack_rows(const void* src, void* dst, const int32_t* b_idx, const int32_t* t_idx,
                             int64_t n_tokens, int heads, int seq, int row_bytes, int mode,
                             hipStream_t stream);
+// Grid of a kernel with one wave per row, `per_group` waves of 64 threads to a group: the groups in
+// x, and in y as well once x alone would pass the 2^32 threads that a launch may have in one
+// dimension (2^26 rows). The kernels take group blockIdx.y * gridDim.x + blockIdx.x and leave the
+// groups past the last row at once.
+constexpr int64_t kRowGroupsX = 1 << 22;
+constexpr int64_t kMaxPaddedRows = (int64_t)1 << 38;
+inline dim3 row_grid(int64_t rows, int per_group) {
+  const int64_t groups = (rows + per_group - 1) / per_group;
+  const int64_t x = groups < kRowGroupsX ? groups : kRowGroupsX;
+  return dim3((unsigned)x, (unsigned)((groups + x - 1) / x));
+}
+
 // row_map (batch * seq) from the tokens' positions; the scatter over it (padded rows without a
 // token become zeros).
 hipError_t launch_row_map(const int32_t* b_idx, const int32_t* t_idx, int64_t n_tokens, int batch,

@@ -360,6 +360,14 @@ def test_attention_entry_points_validate_before_launching():
     assert rc == _lib.VA_EINVAL  # padded layout needs seq > 0
     rc = lib.va_pack_rows(fake, fake, fake, fake, 10, 12, 64, 127, 2, 0, None)
     assert rc == _lib.VA_ESHAPE
+    # padded tensors of 2^31 rows and more pass the size check (the NULL buffers are refused next)
+    rc = lib.va_unpack_rows(None, None, None, None, None, 10, 1 << 20, 1, 1 << 12, 8, 2, None)
+    assert rc == _lib.VA_EINVAL
+    rc = lib.va_rope_fwd_padded(fake, fake, fake, fake, fake, 0, 128, fake, fake, None, fake, fake,
+                                fake, 10, 1 << 20, 1, 1, 128, 1 << 12, 0, 0, None)
+    assert rc == _lib.VA_EINVAL
+    rc = lib.va_unpack_rows(None, None, None, None, None, 10, 1 << 20, 1, 1 << 20, 8, 2, None)
+    assert rc == _lib.VA_ESHAPE
 
 
 def test_product_path_refuses_cpu_tensors():

@@ -192,6 +192,25 @@ def test_row_packing_writes_every_row(batch, seq, n, heads, dim, dtype):
         assert torch.equal(got, ref), fill
 
 
+def test_row_packing_past_2_26_rows():
+    """pack_rows and its backward where one wave per row passes the 2^32 threads of a launch's first
+    dimension: 2^26 and a few rows of 16 bytes, the last tokens and rows among them."""
+    n = (1 << 26) + 6
+    batch, seq, dim = 2, (1 << 25) + 70, 8
+    banner("row packing past 2^26 rows", n, batch, seq)
+    skip = batch * seq - n  # padded rows without a token
+    rows = torch.arange(skip, batch * seq, device="cuda")
+    b, t = (rows // seq).to(torch.int32), (rows % seq).to(torch.int32)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    attn = torch.randint(-99, 99, (batch, 1, seq, dim), generator=gen, device="cuda").half()
+    attn.requires_grad_()
+    out = att.pack_rows(attn, b, t)
+    assert torch.equal(out.detach(), attn.detach().view(-1, dim)[skip:])
+    grad = torch.randint(1, 99, (n, dim), generator=gen, device="cuda").half()
+    back = torch.autograd.grad(out, attn, grad)[0].view(-1, dim)
+    assert torch.equal(back[skip:], grad) and not back[:skip].any()
+
+
 @pytest.mark.parametrize("batch,seq,n,heads,kv_heads,in_dtype", [
     (1, 1, 1, 1, 1, torch.float16), (3, 7, 5, 4, 2, torch.bfloat16),
     (2, 65, 130, 12, 2, torch.float32), (2, 9, 11, 28, 4, torch.float16),
