@@ -171,8 +171,9 @@ def _positions(batch, seq, n, seed):
     (3, 5, 0, 2, 128, torch.float16)])
 def test_row_packing_writes_every_row(batch, seq, n, heads, dim, dtype):
     """pack_rows and its backward at row widths of one chunk, of a power of two and of neither, with
-    rows in any order; the backward's row map scratch and output hold anything before (here a map
-    that names a wrong token for every row)."""
+    rows in any order; the backward's row map scratch and output hold anything before (here NaN, and
+    a map that names no token, a wrong one for every row, or none of the batch's), and the plain
+    scatter of va_pack_rows."""
     banner("row packing", batch, seq, n, heads, dim, dtype)
     b, t = _positions(batch, seq, n, seed=n)
     attn = torch.randn(batch, heads, seq, dim, device="cuda").to(dtype)
@@ -190,6 +191,12 @@ def test_row_packing_writes_every_row(batch, seq, n, heads, dim, dtype):
                   "va_unpack_rows")
         torch.cuda.synchronize()
         assert torch.equal(got, ref), fill
+    got = torch.zeros_like(ref)  # va_pack_rows' own scatter, into a cleared buffer
+    att.check(att.lib().va_pack_rows(grad.data_ptr(), got.data_ptr(), b.data_ptr(), t.data_ptr(), n,
+                                     heads, seq, dim, grad.element_size(), 1, att._stream()),
+              "va_pack_rows")
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref)
 
 
 def test_row_packing_past_2_26_rows():
@@ -211,26 +218,48 @@ def test_row_packing_past_2_26_rows():
     assert torch.equal(back[skip:], grad) and not back[:skip].any()
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("batch,seq,n,heads,kv_heads,in_dtype", [
     (1, 1, 1, 1, 1, torch.float16), (3, 7, 5, 4, 2, torch.bfloat16),
     (2, 65, 130, 12, 2, torch.float32), (2, 9, 11, 28, 4, torch.float16),
     (3, 5, 0, 2, 1, torch.float16)])
-def test_padded_rotation_matches_the_packed_one(batch, seq, n, heads, kv_heads, in_dtype):
-    """qkv_rotate(padded=True) holds the packed rotation's rows, bit for bit, where tokens lie and
-    zeros elsewhere, for rows in any order and outputs from memory that held other values."""
-    banner("padded rotation", batch, seq, n, heads, kv_heads, in_dtype)
+def test_padded_rotation_matches_the_packed_one(batch, seq, n, heads, kv_heads, in_dtype,
+                                                out_dtype):
+    """va_rope_fwd_padded writes the packed rotation's rows, bit for bit, where tokens lie and zeros
+    elsewhere, for rows in any order, into outputs that hold NaN and over a row map that names
+    no token, a wrong token for every row, or none of the batch's; qkv_rotate(padded=True) and
+    va_rope_fwd's padded layout into zeroed outputs give the same."""
+    banner("padded rotation", batch, seq, n, heads, kv_heads, in_dtype, out_dtype)
     b, t = _positions(batch, seq, n, seed=n + 1)
     q = torch.randn(n, heads * 128, device="cuda").to(in_dtype)
     k, v = (torch.randn(n, kv_heads * 128, device="cuda").to(in_dtype) for _ in range(2))
-    cos, sin = torch.randn(batch, seq, 128, device="cuda"), torch.randn(batch, seq, 128, device="cuda")
-    packed = att.qkv_rotate(q, k, v, cos, sin, b, t, batch, seq, heads, kv_heads)
-    junk = torch.full((4 * batch * heads * seq * 128,), float("nan"), device="cuda").half()
-    del junk  # the allocator hands its memory out again
-    padded = att.qkv_rotate(q, k, v, cos, sin, b, t, batch, seq, heads, kv_heads, True)
-    for rows, got in zip(packed, padded):
-        ref = torch.zeros(batch, heads, seq, 128, dtype=torch.float16, device="cuda")
+    cos, sin = (torch.randn(batch, seq, 128, device="cuda") for _ in range(2))
+    refs = []
+    for rows in att.rope_forward(q, k, v, cos, sin, b, t, heads, kv_heads, out_dtype, expand=True):
+        ref = torch.zeros(batch, heads, seq, 128, dtype=out_dtype, device="cuda")
         ref[b.long(), :, t.long()] = rows
-        assert torch.equal(got, ref)
+        refs.append(ref)
+    inputs = [x.data_ptr() for x in (q, k, v, cos, sin)] + [seq * 128, 128, b.data_ptr(),
+                                                            t.data_ptr()]
+    dtypes = [att._DTYPES[in_dtype], att._DTYPES[out_dtype]]
+    for fill in (-1, 0, n - 1, 1 << 30):
+        got = [torch.full_like(ref, float("nan")) for ref in refs]
+        row_map = torch.full((batch * seq,), fill, dtype=torch.int32, device="cuda")
+        att.check(att.lib().va_rope_fwd_padded(*inputs, row_map.data_ptr(),
+                                               *(x.data_ptr() for x in got), n, batch, heads,
+                                               kv_heads, 128, seq, *dtypes, att._stream()),
+                  "va_rope_fwd_padded")
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, ref) for x, ref in zip(got, refs)), fill
+    got = [torch.zeros_like(ref) for ref in refs]
+    att.check(att.lib().va_rope_fwd(*inputs, *(x.data_ptr() for x in got), n, heads, kv_heads, 128,
+                                    seq, *dtypes, att._lib.VA_LAYOUT_PADDED, 1, att._stream()),
+              "va_rope_fwd")
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, ref) for x, ref in zip(got, refs))
+    if out_dtype == torch.float16:
+        got = att.qkv_rotate(q, k, v, cos, sin, b, t, batch, seq, heads, kv_heads, True)
+        assert all(torch.equal(x, ref) for x, ref in zip(got, refs))
 
 
 @pytest.mark.parametrize("heads,kv_heads", [(4, 2), (2, 2)])
