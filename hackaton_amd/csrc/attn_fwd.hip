@@ -716,8 +716,8 @@ __global__ __launch_bounds__(fwdl::NT, fwdl::Ring<KEYS>::PER_CU) void fwd_lean_k
 
   // Read offsets (halfs) inside a tile. K (A operand of S^T): row perm32(l32) (+ 32 b), chunk
   // 2 kk + hi.
-  // V^T: row 8 hi + 2 (src >> 2) + e (+ 16 c + 32 b), chunk 8 (grp & 1) + 2 db + (sg >> 1): registers
-  // [8 c, 8 c + 8) of accumulator db then hold d = 16 db + 64 c + 8 hi + 0..7.
+  // V^T: row 8 hi + 2 (src >> 2) + e (+ 16 c + 32 b), chunk 8 (grp & 1) + 2 db + (sg >> 1):
+  // registers [8 c, 8 c + 8) of accumulator db then hold d = 16 db + 64 c + 8 hi + 0..7.
   int koff[2], toff[2][2];
   {
     const int r = perm32(l32);
@@ -927,8 +927,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a) {
     // 451, at 2600 617 / 627, 521 / 526, 568 / 579, 681 / 682; documents of 16 to 512 at 768 23.3 / 22.0,
     // 22.8 / 21.7, 20.7 / 20.7, 23.7 / 24.8, at 1536 36.6 / 38.4, 34.7 / 36.1, 34.3 / 37.2, 42.2 / 45.2.
     // So short documents would take three from about 1100 items on and long ones lose until 1792;
-    // the sizes that the rule reads do not tell them apart, and below the line the 64-key shape is
-    // at or below the former kernel's time for both.
+    // the sizes that the rule reads do not tell them apart.
     const bool three = (a.n_tokens + fwdl::BM - 1) / fwdl::BM * a.hq >= fwdl::kThreeMinItems;
     hipLaunchKernelGGL((three ? fwd_lean_kernel<E, 32> : fwd_lean_kernel<E, 64>),
                        dim3((unsigned)a.n_items), dim3(fwdl::NT), 0, a.stream,

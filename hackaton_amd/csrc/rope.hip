@@ -256,7 +256,9 @@ __global__ __launch_bounds__(kRopeThreads) void rope_fwd_kernel(RopeArgs a) {
 // The padded layout, every row written once: one wave per padded row (b, t), which holds a token
 // (rotated as above) or zeros. Writing the rows of a zero-filled tensor instead moved the real
 // rows' bytes twice: at 34 rows of 1024 with 18,432 tokens, 12 / 2 heads, fp16, the fills (three
-// 107 MB tensors) and the rotation took 92 us, the row map and this kernel 81 us (396 MB, 4.9 TB/s).
+// 107 MB tensors) and the rotation took 92 us, the row map and this kernel 81 us (396 MB, 4.9 TB/s),
+// repeated alone. Between backwards they take 64 us: the rest of the output leaves the last-level
+// cache during the next kernel (rope_bwd_kernel 42 us alone, 69 after it; 133 us together both ways).
 template <int IN, int OUT>
 __global__ __launch_bounds__(kRopeThreads) void rope_fwd_padded_kernel(RopeArgs a) {
   const long row = grid_row(kTokensPerGroup);
@@ -303,7 +305,8 @@ __device__ inline void bwd_store(const RopeArgs& a, long pid, int b, int t, int 
   const int copies = (!sl.is_q && a.expand) ? a.heads / a.kv_heads : 1;
   // The other copies in batches of 7, every load of a batch issued before its first add: one
   // memory round trip per batch instead of one per copy. (Loading the first batch beside the other
-  // rows of the pass takes 205 registers: 47.5 -> 53 us at 18,432 tokens of 12 / 2 heads, fp16.)
+  // rows of the pass takes 205 registers: 47.5 -> 53 us, each repeated alone, at 18,432 tokens of
+  // 12 / 2 heads, fp16.)
   constexpr int kBatch = 7;
   for (int r0 = 1; r0 < copies; r0 += kBatch) {
     RowIn<IN> more[kBatch];
