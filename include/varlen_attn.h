@@ -147,7 +147,8 @@ int va_stream_capture_id(void* stream, uint64_t* capture_id);
  * From ceil(total_tokens / 128) * Hq >= VA_FWD_MANY_ITEMS on (a lower bound of the list's length
  * that depends on the sizes only, so host and device plans of one batch pick the same kernel)
  * va_fwd runs its many-item kernel (4 waves per item, two work-groups per CU, three from 1792
- * such pairs on) instead of the 8-wave one; both compute the same function (results agree to rounding, each is deterministic).
+ * such pairs on) instead of the 8-wave one; both compute the same function (results agree to
+ * rounding, each is deterministic).
  * va_fwd_kernel is va_fwd with the kernel named: VA_FWD_AUTO (va_fwd's choice), VA_FWD_WIDE (the
  * 8-wave kernel) or VA_FWD_MANY (the many-item kernel), for callers that time or test one of them.
  * Replaces: solution/attention.py:221-222 (aten::_efficient_attention_forward). */
